@@ -67,6 +67,15 @@ GRNS_HD unsigned lane_offset(unsigned v) {
     return v;
 }
 
+// A per-lane 64-bit value kept as one register pair: the optimiser may not take its halves apart
+// (sums whose high word alone is changed stay the addend of the next multiply-add).
+GRNS_HD unsigned long long lane_pair(unsigned long long v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(v));
+#endif
+    return v;
+}
+
 // A view of a constant table (wave-uniform address) whose loads are scalar loads issued where the
 // view is taken: the address goes through uniform_point, and the constant address space lets the
 // compiler use the scalar cache.  On the host it is the plain pointer.  Pass an address computed
@@ -150,7 +159,7 @@ struct DevCtx {
     int pow2_inv[THRESH][MAXN];              // RNS_POW2_INVERSE
     const int *pow2;                         // RNS_POW2, (log2M+1) x n, device memory
     const int *mrc_inv;                      // MRC_MULT_INV, n x n, device memory
-    const double *mrc_inv_d;                 // the same as doubles (per-lane mixed-radix conversion)
+    const int *mrc_acc;                      // n x n: digit sums of the per-lane mixed-radix conversion (lane_mrc)
     int words;                               // 32-bit words of sum_i s_i (M / m_i) < n M
     const unsigned *crt_words;               // (n + 1) x words: M / m_i for i < n, then M
 };

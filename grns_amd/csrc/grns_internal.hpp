@@ -15,7 +15,7 @@ struct grns_ctx {
     grns::DevCtx *d = nullptr;     // device constants
     int *d_pow2 = nullptr;
     int *d_mrc = nullptr;
-    double *d_mrc_d = nullptr;
+    int *d_mrc_acc = nullptr;     // DevCtx::mrc_acc
     int *d_status = nullptr;
     unsigned *d_crt = nullptr;      // DevCtx::crt_words
     int max_blocks = 2048;         // arg-max stage-1 grid, from the occupancy query (max_grid_for)
@@ -48,7 +48,7 @@ struct grns_ctx {
     StageTimer timers[3];
     std::vector<int> pow2;
     std::vector<int> mrc;
-    std::vector<double> mrc_d;
+    std::vector<int> mrc_acc;
     std::vector<unsigned> crt;
 };
 

@@ -1304,52 +1304,67 @@ __global__ __launch_bounds__(FBLOCK) void k_max_final(const DevCtx *__restrict__
 // vector in a column of LDS; the value of a number is that of its residues taken mod m_i, and
 // equal values go to the lower index, so the result is the one grns_max returns.
 
-// Mixed-radix digits of the canonical number held by this lane (mrc, src/mrc.cuh:31-44): step j
-// turns residue i > j into (x_i - d_j) m_j^-1 mod m_i.  Each product is reduced exactly in FP64:
-// with d in (-m_i, m_i) and the inverse in [0, m_i), hi + lo = d * inv exactly (|d * inv| < 2^62);
-// floor(hi / m_i - 2^-19), computed as one fma with RN(1/m_i), is floor(d * inv / m_i) or one less
-// (its error is below 2^-20), so r = d * inv - q m_i is an exact integer in [0, 2 m_i) and one
-// conditional subtraction (an unsigned minimum) ends the reduction.
-// One chunk of step J: residues I0 .. I0 + 3 (those below N).  The constants of the chunk are
-// loaded (scalar loads) once the chunk before the previous one is computed (d2): one chunk of
-// look-ahead rather than the whole table in scalar registers.
-template <int N, int J, int I0>
-GRNS_D void lane_mrc_chunk(const DevCtx *c, const double *tab, int (&mr)[N], int &d1, int &d2) {
-    const DevCtx *cc = reload_after(c, d2);
-    cdouble *inv = const_view(reload_after(tab, d2) + J * N + I0);
-    cdouble *dm = const_view(cc->dm + I0);
-    cdouble *dinv = const_view(cc->dinv + I0);
-    cint *mi = const_view(cc->m + I0);
+// Mixed-radix digits of the canonical number held by this lane (mrc, src/mrc.cuh:31-44).  The
+// reference's steps turn residue i into ((x_i - d_0) m_0^-1 - d_1) m_1^-1 ..., one modular product
+// per (digit, residue) pair; the digit they end at is
+//   d_i = (x_i (m_0 ... m_{i-1})^-1 - sum_{k < i} d_k (m_k ... m_{i-1})^-1) mod m_i,
+// one sum of i + 1 products with constants (row i of the table, negated for k < i) and one
+// reduction.  A product is one v_mad_u64_u32 (it issues at the rate of an FP64 operation on this
+// chip); after every two products the sum's high word is reduced by one conditional subtraction of
+// m_i (a multiple of m_i 2^32), which keeps the sum below 2^64: with hi < m_i < 2^31 before, two
+// products below 2^31 m_i each leave hi < 2 m_i.  The digits are unique, so they are the
+// reference's.  About 2.5 instructions per pair, where a modular product per pair takes 11 FP64
+// operations: 2e6 numbers of 32 moduli convert in 150 us instead of 326 us (3.4 TB/s of loads and
+// stores together).
+
+// Terms C0 .. C0 + 15 (those up to I) of digit I.  The constants are loaded (scalar loads) once the
+// chunk before the previous one is computed (d2): one chunk of look-ahead rather than the whole
+// table in scalar registers.
+constexpr int MRC_CHUNK = 16;
+template <int N, int I, int C0>
+GRNS_D void lane_mrc_chunk(const int *tab, const int (&mr)[N], unsigned m, unsigned long long &acc, int &d1, int &d2) {
+    cint *t = const_view(reload_after(tab, d2) + I * N + C0);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (I0 + k < N) {
-            const double d = (double)(mr[I0 + k] - mr[J]);
-            const double hi = d * inv[k];
-            const double lo = fma(d, inv[k], -hi);
-            const double q = floor(fma(hi, dinv[k], -0x1p-19));
-            const unsigned r = (unsigned)(fma(-q, dm[k], hi) + lo);
-            const unsigned s = r - (unsigned)mi[k];
-            mr[I0 + k] = (int)(s < r ? s : r);
+    for (int k = 0; k < MRC_CHUNK; k++) {
+        if (C0 + k <= I) {
+            acc += (unsigned long long)(unsigned)mr[C0 + k] * (unsigned)t[k];
+            if ((C0 + k) % 2 == 1 || C0 + k == I) {
+                const unsigned hi = (unsigned)(acc >> 32), h2 = hi - m;
+                acc = lane_pair(((unsigned long long)(h2 < hi ? h2 : hi) << 32) | (unsigned)acc);
+            }
         }
     }
     d2 = d1;
-    d1 = mr[I0 + 3 < N ? I0 + 3 : N - 1];
+    d1 = (int)(unsigned)acc;
 }
-template <int N, int J, int... C>
-GRNS_D void lane_mrc_step(const DevCtx *c, const double *tab, int (&mr)[N], int &d1, int &d2,
-                          std::integer_sequence<int, C...>) {
-    (lane_mrc_chunk<N, J, J + 1 + 4 * C>(c, tab, mr, d1, d2), ...);
+// The sum (hi < m) mod m: its quotient, below 2^32, comes from a double within 2^-18 of sum / m
+// that is biased down by as much, so it is the true one or one less.
+GRNS_D int mrc_reduce(unsigned long long acc, unsigned m, double dinv) {
+    const double v = fma((double)(unsigned)(acc >> 32), 4294967296.0, (double)(unsigned)acc);
+    const unsigned q = (unsigned)fma(v, dinv, -0x1p-18);
+    const unsigned r = (unsigned)acc - q * m, s = r - m;
+    return (int)(s < r ? s : r);
 }
-template <int N, int... J>
-GRNS_D void lane_mrc_steps(const DevCtx *c, const double *tab, int (&mr)[N], std::integer_sequence<int, J...>) {
-    int d1 = 0, d2 = 0;
-    (lane_mrc_step<N, J>(c, tab, mr, d1, d2, std::make_integer_sequence<int, (N - 1 - J + 3) / 4>{}), ...);
+template <int N, int I, int... C>
+GRNS_D void lane_mrc_digit(const DevCtx *c, const int *tab, int (&mr)[N], int &d1, int &d2,
+                           std::integer_sequence<int, C...>) {
+    const DevCtx *cc = reload_after(c, d2);
+    const unsigned m = (unsigned)const_view(cc->m + I)[0];
+    const double dinv = const_view(cc->dinv + I)[0];
+    unsigned long long acc = 0;
+    (lane_mrc_chunk<N, I, MRC_CHUNK * C>(tab, mr, m, acc, d1, d2), ...);
+    mr[I] = mrc_reduce(acc, m, dinv);
 }
-// Every step, as straight-line code (all register indexes are constants).  tab: the context's
-// inverse table as doubles (c->mrc_inv_d), read once by the caller.
+template <int N, int... I>
+GRNS_D void lane_mrc_digits(const DevCtx *c, const int *tab, int (&mr)[N], std::integer_sequence<int, I...>) {
+    int d1 = 0, d2 = 0;  // digit 0 is residue 0
+    (lane_mrc_digit<N, I + 1>(c, tab, mr, d1, d2, std::make_integer_sequence<int, (I + 1) / MRC_CHUNK + 1>{}), ...);
+}
+// Every digit, as straight-line code (all register indexes are constants).  tab: the context's
+// table (c->mrc_acc), read once by the caller.
 template <int N>
-GRNS_D void lane_mrc(const DevCtx *c, const double *tab, int (&mr)[N]) {
-    lane_mrc_steps<N>(c, tab, mr, std::make_integer_sequence<int, N - 1>{});
+GRNS_D void lane_mrc(const DevCtx *c, const int *tab, int (&mr)[N]) {
+    lane_mrc_digits<N>(c, tab, mr, std::make_integer_sequence<int, N - 1>{});
 }
 
 // Order of the digit vector `a` (this lane's registers) against column `col` of `bd` below the top
@@ -1390,7 +1405,7 @@ __global__ __launch_bounds__(BLOCK) void k_max_mrc_partial(const DevCtx *__restr
     const int t = threadIdx.x;
     const long long start = (long long)blockIdx.x * chunk;
     const long long end = start + chunk < count ? start + chunk : count;
-    const double *tab = c->mrc_inv_d;
+    const int *tab = c->mrc_acc;
     long long best = -1;
     int top = 0;
     for (long long b0 = start; b0 < end; b0 += BLOCK) {
@@ -1810,7 +1825,7 @@ template <int N>
 __global__ __launch_bounds__(BLOCK) void k_mrc_lane(const DevCtx *__restrict__ c, const int *__restrict__ x,
                                                     long long smod, long long snum, long long count,
                                                     int *__restrict__ d, long long dsm, long long dsn) {
-    const double *tab = c->mrc_inv_d;
+    const int *tab = c->mrc_acc;
     for (long long base = (long long)blockIdx.x * BLOCK; base < count; base += (long long)gridDim.x * BLOCK) {
         const long long j = base + threadIdx.x;
         bool coop = false;

@@ -180,7 +180,16 @@ grns_status build_constants(grns_ctx *c, const int *moduli, int n) {
     c->mrc.assign((size_t)n * n, 0);
     for (int i = 0; i < n; i++)
         for (int j = i + 1; j < n; j++) c->mrc[(size_t)i * n + j] = inverse_mod(moduli[i], moduli[j]);
-    c->mrc_d.assign(c->mrc.begin(), c->mrc.end());
+    // Row i of mrc_acc: -(m_k ... m_{i-1})^-1 mod m_i at k < i, and (m_0 ... m_{i-1})^-1 at k = i
+    c->mrc_acc.assign((size_t)n * n, 0);
+    for (int i = 0; i < n; i++) {
+        long long inv = 1 % moduli[i];
+        for (int k = i - 1; k >= 0; k--) {
+            inv = inv * c->mrc[(size_t)k * n + i] % moduli[i];
+            c->mrc_acc[(size_t)i * n + k] = (int)((moduli[i] - inv) % moduli[i]);
+        }
+        c->mrc_acc[(size_t)i * n + i] = (int)inv;
+    }
     // M / m_i and M as 32-bit words, one word more than M has (room for sum_i s_i M / m_i < n M)
     const int WW = (int)limbs.size() + 1;
     h.words = WW;
@@ -423,19 +432,19 @@ grns_status grns_ctx_create(const int *moduli, int n, int device, grns_ctx **out
         hipMalloc(&c->d_crt, sizeof(unsigned) * c->crt.size()) != hipSuccess ||
         hipMalloc(&c->d_pow2, sizeof(int) * c->pow2.size()) != hipSuccess ||
         hipMalloc(&c->d_mrc, sizeof(int) * c->mrc.size()) != hipSuccess ||
-        hipMalloc(&c->d_mrc_d, sizeof(double) * c->mrc_d.size()) != hipSuccess ||
+        hipMalloc(&c->d_mrc_acc, sizeof(int) * c->mrc_acc.size()) != hipSuccess ||
         hipMalloc(&c->d_status, sizeof(int)) != hipSuccess) {
         grns_ctx_destroy(c);
         return GRNS_ERR_OOM;
     }
     c->h.pow2 = c->d_pow2;
     c->h.mrc_inv = c->d_mrc;
-    c->h.mrc_inv_d = c->d_mrc_d;
+    c->h.mrc_acc = c->d_mrc_acc;
     c->h.crt_words = c->d_crt;
     if (hipMemcpy(c->d_crt, c->crt.data(), sizeof(unsigned) * c->crt.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_pow2, c->pow2.data(), sizeof(int) * c->pow2.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_mrc, c->mrc.data(), sizeof(int) * c->mrc.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->d_mrc_d, c->mrc_d.data(), sizeof(double) * c->mrc_d.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->d_mrc_acc, c->mrc_acc.data(), sizeof(int) * c->mrc_acc.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d, &c->h, sizeof(DevCtx), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(c->d_status, 0, sizeof(int)) != hipSuccess ||
         hipDeviceSynchronize() != hipSuccess) {  // tables and status in place before any stream's kernels
@@ -459,7 +468,7 @@ grns_status grns_ctx_destroy(grns_ctx *c) {
         if (c->d_pow2) (void)hipFree(c->d_pow2);
         if (c->d_crt) (void)hipFree(c->d_crt);
         if (c->d_mrc) (void)hipFree(c->d_mrc);
-        if (c->d_mrc_d) (void)hipFree(c->d_mrc_d);
+        if (c->d_mrc_acc) (void)hipFree(c->d_mrc_acc);
         if (c->d_status) (void)hipFree(c->d_status);
         for (auto &q : c->queues) {
             (void)hipFree(q.items);
@@ -1134,7 +1143,7 @@ DevCtx host_view(const grns_ctx *c) {
     DevCtx h = c->h;
     h.pow2 = c->pow2.data();
     h.mrc_inv = c->mrc.data();
-    h.mrc_inv_d = c->mrc_d.data();
+    h.mrc_acc = c->mrc_acc.data();
     h.crt_words = c->crt.data();
     return h;
 }
