@@ -80,13 +80,16 @@ GRNS_D bool next_tile(const BatchTask *__restrict__ tasks, int ntasks, long long
     return t < total;
 }
 
-// Operation class of a thread-mapped task list: one kernel instantiation per class, so that each
-// carries only its class's code and runs with its registers and occupancy (as the per-call kernels
-// do): evaluation (and its fast form), comparison, and the mpint add / sub / mul, whose codes need
-// about the same registers (104-114 VGPRs at n = 32) and so share one kernel and one tile space.
-enum : int { OPS_EVAL = 1, OPS_CMP = 2, OPS_MPINT = 4 };
-constexpr int OP_CLASSES = 3;
-constexpr int BATCH_COUNTERS = 4;  // tile counters: one per thread list (3), one for the group list
+// Operation class of a task list: one kernel instantiation per class, so that each carries only its
+// class's code and runs with its registers and occupancy (as the per-call kernels do).  Lane per
+// number: evaluation (and its fast form), comparison, and the mpint add / sub / mul, whose codes
+// need about the same registers (104-114 VGPRs at n = 32) and so share one kernel and one tile
+// space.  Wave group per number: division, scaling, and the element-wise operations of layouts and
+// moduli counts without a lane form.  (One kernel for all group operations took the registers of
+// the largest, 174 VGPRs and two waves per SIMD.)
+enum : int { OPS_EVAL = 1, OPS_CMP = 2, OPS_MPINT = 4, OPS_DIV = 8, OPS_SCALE = 16, OPS_GROUP = 32 };
+constexpr int OP_CLASSES = 6;
+constexpr int BATCH_COUNTERS = OP_CLASSES;  // a tile counter per list
 
 template <int N, int OPS>
 __global__ __launch_bounds__(BLOCK) void k_batch_thread(const DevCtx *__restrict__ c, const BatchTask *__restrict__ tasks,
@@ -135,10 +138,12 @@ __global__ __launch_bounds__(BLOCK) void k_batch_thread(const DevCtx *__restrict
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_batch_group(const DevCtx *__restrict__ c, int G,
-                                                       const BatchTask *__restrict__ tasks, int ntasks, long long total,
-                                                       int tile, unsigned long long *counter, int *__restrict__ status) {
-    Group g = make_group(G, c->n);
+// The numbers of the tiles of a group list: body(T, g, j) for every number j of every tile the block
+// takes, a group of G lanes per number.
+template <class Body>
+GRNS_D void for_group_tiles(const DevCtx *c, int G, const BatchTask *__restrict__ tasks, int ntasks, long long total,
+                            int tile, unsigned long long *counter, Body body) {
+    const Group g = make_group(G, c->n);
     const int P = 64 / G;
     const long long wave = threadIdx.x >> 6;
     const long long gid = (threadIdx.x & 63) / G;
@@ -146,80 +151,87 @@ __global__ __launch_bounds__(BLOCK) void k_batch_group(const DevCtx *__restrict_
     int k;
     while (next_tile(tasks, ntasks, total, counter, t, k)) {
         const BatchTask &T = tasks[k];
-        long long e0 = (t - T.tile0) * tile;
-        long long e1 = e0 + tile < T.count ? e0 + tile : T.count;
+        const long long e0 = (t - T.tile0) * tile;
+        const long long e1 = e0 + tile < T.count ? e0 + tile : T.count;
         for (long long j0 = e0 + wave * P; j0 < e1; j0 += (BLOCK / 64) * P) {
-            long long j = j0 + gid;
-            if (j >= e1) continue;
-            int st = 0;
-            const bool act = g.gl < g.L;
-            long long oa = j * T.asn + (long long)g.gl * T.asm_;
-            switch (T.op) {
-                case GRNS_OP_EVAL:
-                case GRNS_OP_EVAL_FAST: {
-                    int xi = act ? T.a[oa] : 0;
-                    interval_t r = (T.op == GRNS_OP_EVAL) ? group_eval<false>(c, g, xi, st) : group_eval<true>(c, g, xi, st);
-                    if (g.gl == 0) store_interval(reinterpret_cast<interval_t *>(T.o0) + j, r);
-                    break;
-                }
-                case GRNS_OP_CMP: {
-                    int xi = act ? T.a[oa] : 0;
-                    int yi = act ? T.b[j * T.bsn + (long long)g.gl * T.bsm] : 0;
-                    int r = group_cmp(c, g, xi, yi, st);
-                    if (g.gl == 0) reinterpret_cast<int *>(T.o0)[j] = r;
-                    break;
-                }
-                case GRNS_OP_MPINT_ADD: group_mpint<0>(c, g, T.mp, j); break;
-                case GRNS_OP_MPINT_SUB: group_mpint<1>(c, g, T.mp, j); break;
-                case GRNS_OP_MPINT_MUL: group_mpint<2>(c, g, T.mp, j); break;
-                case GRNS_OP_DIV:
-                case GRNS_OP_DIV_FAST: {
-                    int xi = act ? T.a[oa] : 0;
-                    int di = act ? T.b[oa] : 0;
-                    int q, r;
-                    if (g.G >= c->words && g.G >= 4 && div_words_ok(c, g, xi, di)) {
-                        switch (g.G) {
-                            case 4: group_div_words<4>(c, g, xi, di, q, r); break;
-                            case 8: group_div_words<8>(c, g, xi, di, q, r); break;
-                            case 16: group_div_words<16>(c, g, xi, di, q, r); break;
-                            case 32: group_div_words<32>(c, g, xi, di, q, r); break;
-                            default: group_div_words<64>(c, g, xi, di, q, r); break;
-                        }
-                    } else if (T.op == GRNS_OP_DIV) {
-                        group_div<false>(c, g, xi, di, q, r, st);
-                    } else {
-                        group_div<true>(c, g, xi, di, q, r, st);
-                    }
-                    if (act) {
-                        reinterpret_cast<int *>(T.o0)[oa] = q;
-                        reinterpret_cast<int *>(T.o1)[oa] = r;
-                    }
-                    break;
-                }
-                case GRNS_OP_SCALE2POW: {
-                    int xi = act ? T.a[oa] : 0;
-                    const unsigned Dj = T.D[j];
-                    bool ok = false;
-                    int v = 0;
-                    if (g.G >= c->words && g.G >= 4 && group_all(g, !act || (unsigned)xi < (unsigned)c->m[g.gl])) {
-                        switch (g.G) {
-                            case 4: v = group_scale2pow_words<4>(c, g, xi, Dj, ok); break;
-                            case 8: v = group_scale2pow_words<8>(c, g, xi, Dj, ok); break;
-                            case 16: v = group_scale2pow_words<16>(c, g, xi, Dj, ok); break;
-                            case 32: v = group_scale2pow_words<32>(c, g, xi, Dj, ok); break;
-                            default: v = group_scale2pow_words<64>(c, g, xi, Dj, ok); break;
-                        }
-                    }
-                    if (!ok) v = group_scale2pow(c, g, xi, Dj);
-                    if (act) reinterpret_cast<int *>(T.o0)[oa] = v;
-                    break;
-                }
-                default:
-                    break;
-            }
-            if (g.gl == 0 && st) atomicOr(status, st);
+            const long long j = j0 + gid;
+            if (j < e1) body(T, g, j);
         }
     }
+}
+
+// Division (group of GD lanes per pair): the word division, or the reference loop for the pairs it
+// does not take.
+template <int GD>
+__global__ __launch_bounds__(BLOCK) void k_batch_div(const DevCtx *__restrict__ c, const BatchTask *__restrict__ tasks,
+                                                     int ntasks, long long total, int tile,
+                                                     unsigned long long *counter, int *__restrict__ status) {
+    for_group_tiles(c, GD, tasks, ntasks, total, tile, counter, [&](const BatchTask &T, const Group &g, long long j) {
+        const bool act = g.gl < g.L;
+        const long long oa = j * T.asn + (long long)g.gl * T.asm_;
+        const int xi = act ? T.a[oa] : 0;
+        const int di = act ? T.b[oa] : 0;
+        int q, r, st = 0;
+        if (div_words_ok(c, g, xi, di)) group_div_words<GD>(c, g, xi, di, q, r);
+        else if (T.op == GRNS_OP_DIV) group_div<false>(c, g, xi, di, q, r, st);
+        else group_div<true>(c, g, xi, di, q, r, st);
+        if (act) {
+            reinterpret_cast<int *>(T.o0)[oa] = q;
+            reinterpret_cast<int *>(T.o1)[oa] = r;
+        }
+        if (g.gl == 0 && st) atomicOr(status, st);
+    });
+}
+
+// Scaling (group of GD lanes per number): the replay, or the reference steps for the numbers it
+// does not take.
+template <int GD>
+__global__ __launch_bounds__(BLOCK) void k_batch_scale(const DevCtx *__restrict__ c,
+                                                       const BatchTask *__restrict__ tasks, int ntasks,
+                                                       long long total, int tile, unsigned long long *counter) {
+    for_group_tiles(c, GD, tasks, ntasks, total, tile, counter, [&](const BatchTask &T, const Group &g, long long j) {
+        const bool act = g.gl < g.L;
+        const long long oa = j * T.asn + (long long)g.gl * T.asm_;
+        const int xi = act ? T.a[oa] : 0;
+        const unsigned Dj = T.D[j];
+        bool ok = false;
+        int v = 0;
+        if (group_all(g, !act || (unsigned)xi < (unsigned)c->m[g.gl])) v = group_scale2pow_words<GD>(c, g, xi, Dj, ok);
+        if (!ok) v = group_scale2pow(c, g, xi, Dj);
+        if (act) reinterpret_cast<int *>(T.o0)[oa] = v;
+    });
+}
+
+// The element-wise operations by groups.
+__global__ __launch_bounds__(BLOCK) void k_batch_group(const DevCtx *__restrict__ c, int G,
+                                                       const BatchTask *__restrict__ tasks, int ntasks, long long total,
+                                                       int tile, unsigned long long *counter, int *__restrict__ status) {
+    for_group_tiles(c, G, tasks, ntasks, total, tile, counter, [&](const BatchTask &T, const Group &g, long long j) {
+        int st = 0;
+        const bool act = g.gl < g.L;
+        const long long oa = j * T.asn + (long long)g.gl * T.asm_;
+        switch (T.op) {
+            case GRNS_OP_EVAL:
+            case GRNS_OP_EVAL_FAST: {
+                int xi = act ? T.a[oa] : 0;
+                interval_t r = (T.op == GRNS_OP_EVAL) ? group_eval<false>(c, g, xi, st) : group_eval<true>(c, g, xi, st);
+                if (g.gl == 0) store_interval(reinterpret_cast<interval_t *>(T.o0) + j, r);
+                break;
+            }
+            case GRNS_OP_CMP: {
+                int xi = act ? T.a[oa] : 0;
+                int yi = act ? T.b[j * T.bsn + (long long)g.gl * T.bsm] : 0;
+                int r = group_cmp(c, g, xi, yi, st);
+                if (g.gl == 0) reinterpret_cast<int *>(T.o0)[j] = r;
+                break;
+            }
+            case GRNS_OP_MPINT_ADD: group_mpint<0>(c, g, T.mp, j); break;
+            case GRNS_OP_MPINT_SUB: group_mpint<1>(c, g, T.mp, j); break;
+            case GRNS_OP_MPINT_MUL: group_mpint<2>(c, g, T.mp, j); break;
+            default: break;
+        }
+        if (g.gl == 0 && st) atomicOr(status, st);
+    });
 }
 
 __global__ void k_batch_reset(unsigned long long *counters) {
@@ -259,25 +271,31 @@ BatchTask to_dev(const grns_batch_task &u) {
     return t;
 }
 
-// Tasks split by mapping and operation: the thread-per-number lists first, one per operation, then
-// the group-per-number list; each list has its own tile prefix (tile0 counts from 0 within it).
-struct ThreadList {
+// Tasks split by mapping and operation, one list per class; each list has its own tile prefix
+// (tile0 counts from 0 within it).  Tiles of the group classes are 16 times smaller: a group does
+// far more work per number.
+struct TaskList {
     int ops;          // OPS_* of the list's operation
     int first;        // index of its first task in TaskPlan::all
     int count;        // tasks
-    long long tiles;  // tiles of `tile` numbers
+    int tile;         // numbers per tile
+    long long tiles;
 };
 
 struct TaskPlan {
     std::vector<BatchTask> all;
-    std::vector<ThreadList> lists;
-    int nthr = 0, ngrp = 0;
-    long long grp_tiles = 0;
-    long long grp_tile = 1;  // numbers per tile of the group list: a group does far more work per number
+    std::vector<TaskList> lists;
 };
 
-int op_class(int op) {
-    switch (op) {
+int op_class(const grns_batch_task &u, bool thread_ok) {
+    switch (u.op) {
+        case GRNS_OP_DIV:
+        case GRNS_OP_DIV_FAST: return OPS_DIV;
+        case GRNS_OP_SCALE2POW: return OPS_SCALE;
+        default: break;
+    }
+    if (!thread_ok || !lane_layout(u)) return OPS_GROUP;
+    switch (u.op) {
         case GRNS_OP_EVAL:
         case GRNS_OP_EVAL_FAST: return OPS_EVAL;
         case GRNS_OP_CMP: return OPS_CMP;
@@ -288,25 +306,16 @@ int op_class(int op) {
 void make_plan(const grns_batch_task *u, int n, int ctx_n, const grns_batch_config &cfg, TaskPlan &P) {
     P.all.clear();
     P.lists.clear();
-    std::vector<BatchTask> grp, by_op[OP_CLASSES];
+    std::vector<BatchTask> by_op[OP_CLASSES];
     const bool thread_ok = thread_kernel_available(ctx_n) && cfg.threads_per_number == 1;
-    const long long tile = cfg.tile;
-    P.grp_tile = tile / 16 > 0 ? tile / 16 : 1;
-    P.grp_tiles = 0;
     for (int i = 0; i < n; i++) {
         if (u[i].count == 0 || u[i].op == GRNS_OP_MAX) continue;
-        BatchTask t = to_dev(u[i]);
-        if (thread_ok && elementwise(u[i].op) && lane_layout(u[i])) {
-            by_op[__builtin_ctz(op_class(u[i].op))].push_back(t);
-        } else {
-            t.tile0 = P.grp_tiles;
-            P.grp_tiles += (t.count + P.grp_tile - 1) / P.grp_tile;
-            grp.push_back(t);
-        }
+        by_op[__builtin_ctz(op_class(u[i], thread_ok))].push_back(to_dev(u[i]));
     }
     for (int k = 0; k < OP_CLASSES; k++) {
         if (by_op[k].empty()) continue;
-        ThreadList L{1 << k, (int)P.all.size(), (int)by_op[k].size(), 0};
+        const int tile = (1 << k) >= OPS_DIV ? (cfg.tile / 16 > 0 ? cfg.tile / 16 : 1) : cfg.tile;
+        TaskList L{1 << k, (int)P.all.size(), (int)by_op[k].size(), tile, 0};
         for (BatchTask &t : by_op[k]) {
             t.tile0 = L.tiles;
             L.tiles += (t.count + tile - 1) / tile;
@@ -314,54 +323,73 @@ void make_plan(const grns_batch_task *u, int n, int ctx_n, const grns_batch_conf
         }
         P.lists.push_back(L);
     }
-    P.nthr = (int)P.all.size();
-    P.ngrp = (int)grp.size();
-    P.all.insert(P.all.end(), grp.begin(), grp.end());
 }
 
-// Counter reset plus one persistent launch per non-empty list, in order on the stream; d_tasks
-// must hold P.all.
 template <int NN>
-void launch_thread_list(grns_ctx *c, const ThreadList &L, const BatchTask *d_tasks, unsigned long long *counter,
-                        int tile, dim3 grid, hipStream_t s) {
+void launch_thread_list(grns_ctx *c, const TaskList &L, const BatchTask *tl, unsigned long long *counter, dim3 grid,
+                        hipStream_t s) {
     const dim3 blk(BLOCK);
-    const BatchTask *tl = d_tasks + L.first;
     switch (L.ops) {
         case OPS_EVAL:
-            hipLaunchKernelGGL((k_batch_thread<NN, OPS_EVAL>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, tile, counter,
-                               c->d_status);
+            hipLaunchKernelGGL((k_batch_thread<NN, OPS_EVAL>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, L.tile,
+                               counter, c->d_status);
             break;
         case OPS_CMP:
-            hipLaunchKernelGGL((k_batch_thread<NN, OPS_CMP>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, tile, counter,
-                               c->d_status);
+            hipLaunchKernelGGL((k_batch_thread<NN, OPS_CMP>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, L.tile,
+                               counter, c->d_status);
             break;
         default:
-            hipLaunchKernelGGL((k_batch_thread<NN, OPS_MPINT>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, tile,
+            hipLaunchKernelGGL((k_batch_thread<NN, OPS_MPINT>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, L.tile,
                                counter, c->d_status);
             break;
     }
 }
 
+// Division or scaling with the word forms' group width.
+template <int GD>
+void launch_words_list(grns_ctx *c, const TaskList &L, const BatchTask *tl, unsigned long long *counter, dim3 grid,
+                       hipStream_t s) {
+    const dim3 blk(BLOCK);
+    if (L.ops == OPS_DIV)
+        hipLaunchKernelGGL((k_batch_div<GD>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, L.tile, counter, c->d_status);
+    else
+        hipLaunchKernelGGL((k_batch_scale<GD>), grid, blk, 0, s, c->d, tl, L.count, L.tiles, L.tile, counter);
+}
+
+// Counter reset plus one persistent launch per non-empty list, in order on the stream; d_tasks
+// must hold P.all.
 grns_status enqueue_plan(grns_ctx *c, const TaskPlan &P, const BatchTask *d_tasks, unsigned long long *d_counters,
                          const grns_batch_config &cfg, int cus, hipStream_t s) {
     hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, d_counters);
     dim3 grid((unsigned)(cus * cfg.blocks_per_cu)), blk(BLOCK);
     for (size_t li = 0; li < P.lists.size(); li++) {
         unsigned long long *counter = d_counters + li;
-        switch (c->n) {
-            case 4: launch_thread_list<4>(c, P.lists[li], d_tasks, counter, cfg.tile, grid, s); break;
-            case 8: launch_thread_list<8>(c, P.lists[li], d_tasks, counter, cfg.tile, grid, s); break;
-            case 16: launch_thread_list<16>(c, P.lists[li], d_tasks, counter, cfg.tile, grid, s); break;
-            case 32: launch_thread_list<32>(c, P.lists[li], d_tasks, counter, cfg.tile, grid, s); break;
-            case 64: launch_thread_list<64>(c, P.lists[li], d_tasks, counter, cfg.tile, grid, s); break;
-            default: return GRNS_ERR_UNSUPPORTED;
+        const TaskList &L = P.lists[li];
+        const BatchTask *tl = d_tasks + L.first;
+        if (L.ops == OPS_GROUP) {
+            const int G = groups_for(c->n);
+            hipLaunchKernelGGL(k_batch_group, grid, blk, 0, s, c->d, G, tl, L.count, L.tiles, L.tile, counter,
+                               c->d_status);
+        } else if (L.ops == OPS_DIV || L.ops == OPS_SCALE) {
+            switch (words_group(c)) {  // every set of up to 64 moduli has a word form
+                case 2: launch_words_list<2>(c, L, tl, counter, grid, s); break;
+                case 4: launch_words_list<4>(c, L, tl, counter, grid, s); break;
+                case 8: launch_words_list<8>(c, L, tl, counter, grid, s); break;
+                case 16: launch_words_list<16>(c, L, tl, counter, grid, s); break;
+                case 32: launch_words_list<32>(c, L, tl, counter, grid, s); break;
+                case 64: launch_words_list<64>(c, L, tl, counter, grid, s); break;
+                default: return GRNS_ERR_UNSUPPORTED;
+            }
+        } else {
+            switch (c->n) {
+                case 4: launch_thread_list<4>(c, L, tl, counter, grid, s); break;
+                case 8: launch_thread_list<8>(c, L, tl, counter, grid, s); break;
+                case 16: launch_thread_list<16>(c, L, tl, counter, grid, s); break;
+                case 32: launch_thread_list<32>(c, L, tl, counter, grid, s); break;
+                case 64: launch_thread_list<64>(c, L, tl, counter, grid, s); break;
+                default: return GRNS_ERR_UNSUPPORTED;
+            }
         }
-    }
-    if (P.ngrp) {
-        // group width: the word division's when it has one (the group tasks are mostly divisions)
-        const int G = words_group(c) ? words_group(c) : groups_for(c->n);
-        hipLaunchKernelGGL(k_batch_group, grid, blk, 0, s, c->d, G, d_tasks + P.nthr, P.ngrp,
-                           P.grp_tiles, (int)P.grp_tile, d_counters + BATCH_COUNTERS - 1, c->d_status);
     }
     return hipGetLastError() == hipSuccess ? GRNS_OK : GRNS_ERR_HIP;
 }

@@ -152,6 +152,12 @@ struct DevCtx {
     double shi[MAXN];            // as khi, klo for (2^KEY_SHIFT w_i mod m_i) / m_i: the key of
     double slo[MAXN];            //   2^KEY_SHIFT x, for values within 2^-28 M of 0 or M
     int c32[MAXN];               // 2^32 mod m_i
+    int odd_moduli;              // 1 when every m_i is odd (scaling steps by exact division)
+    unsigned minv[MAXN];         // m_i^-1 mod 2^32 (odd m_i)
+    unsigned wf_hi[MAXN];        // floor(2^64 w_i / m_i): the fraction of y w_i / m_i for y < 2^32
+    unsigned wf_lo[MAXN];
+    unsigned rec_t[MAXN];        // residues y in [rec_t, rec_t + rec_lim) are far enough from 0 and m_i
+    unsigned rec_lim[MAXN];      //   that every reciprocal reduction giving y is canonical
     unsigned long long mi64[MAXN];  // (M / m_i) mod 2^64
     unsigned long long M64;         // M mod 2^64
     int prod_pow2_res[THRESH];               // RNS_MODULI_PRODUCT_POW2_RESIDUES
@@ -1127,6 +1133,38 @@ GRNS_D void group_div_words(const DevCtx *c, const Group &g, int xi, int di, int
     }
 }
 
+// One step of the replay below as the reference computes it, for any y it may hold: X_s mod 2^j is
+// r, inv is (2^j)^-1 mod m.  `bad`: c = y w is not canonical, or y' wraps int32.
+GRNS_D int scale_step_reference(int y, unsigned r, int w, int inv, int m, double dinv, bool &bad) {
+    const int cc = mulmod_recip(y, w, m, dinv);
+    bad |= (unsigned)cc >= (unsigned)m;
+    // rm = r % m and mult = (y - rm + m) % m as rem_trunc forms them: r < 2^30 and
+    // |y - rm + m| < 2^32 have exact doubles, formed from 32-bit pieces
+    const int rm = (int)rem_trunc_d((long long)r, (double)r, m, dinv);
+    const int mult = (int)rem_trunc_d((long long)y + (m - rm), (double)y + (double)(m - rm), m, dinv);
+    const int qi = (int)(((double)mult * (double)inv) * dinv);
+    const long long v = (long long)mult * inv - (long long)qi * m;
+    bad |= v < -2147483648ll || v > 2147483647ll;
+    return (int)v;
+}
+
+// Bits [30 l, 30 l + 30) of the group's value, l >= 0 the lane's own choice.
+template <int GD>
+GRNS_D unsigned digit30(const Group &g, unsigned X, int l) {
+    const int b = 30 * l, w0 = b >> 5, sh = b & 31;
+    unsigned lo = (unsigned)__shfl((int)X, g.base + (w0 < GD ? w0 : 0), 64);
+    unsigned hi = (unsigned)__shfl((int)X, g.base + (w0 + 1 < GD ? w0 + 1 : 0), 64);
+    lo = w0 < GD ? lo : 0u;
+    hi = w0 + 1 < GD ? hi : 0u;
+    return (unsigned)((((unsigned long long)hi << 32) | lo) >> sh) & 0x3fffffffu;
+}
+
+// The active lanes whose y' (yo = y' - rec_t) or fraction f of y w / m (32 bits, at most 2 below
+// the true one) is too near the edges: both limits keep a fraction 2^-20 from an integer.
+GRNS_D unsigned long long scale_edges(unsigned yo, unsigned ylim, unsigned f) {
+    return __builtin_amdgcn_uicmp(yo, ylim, 35) | __builtin_amdgcn_uicmp(f - 4100u, 0u - 8200u, 35);  // ICMP_UGE
+}
+
 // rns_scale2pow (src/rnsscal.cuh:93-119) replayed on the words of a canonical x.  Step s of the
 // reference maps its value X_s = floor(x / 2^(30 s)) to X_{s+1} = floor(X_s / 2^j): with its
 // residues y (as the reference holds them, possibly y + m or y - m) it forms c = y * w (for the
@@ -1136,43 +1174,71 @@ GRNS_D void group_div_words(const DevCtx *c, const Group &g, int xi, int di, int
 // of x, and y' follows from y exactly as the reference computes it.  A step whose c is not
 // canonical or whose y' wraps int32 (the reference then continues with another number) sets
 // `replay_ok` false and the caller runs the reference steps instead.
+//
+// A reciprocal product is canonical unless its fraction is within 2^-20.4 of an integer.  So a step
+// from canonical y first takes its y' by exact division, y' = (y - r) / 2^j mod m = (d - h m) / 2^j
+// with d = y - r and h = d m^-1 mod 2^j (two 32-bit multiplications: the low parts of d and h m are
+// equal, so the high parts alone give the quotient), and the fraction of y w / m to 32 bits (two
+// more): when every lane's y' and fraction keep their distance from the edges, the reference's
+// products are canonical and y' is its result.  Otherwise the step (one in about 10^4, and those
+// near the end of a small value) runs as the reference computes it; so does every step of a set
+// with an even modulus, which has no inverse of 2.  13 vector instructions per step instead of 64:
+// 2^20 numbers of 64 moduli with D uniform in [1, 1900] take 2.3 ms instead of 5.0 ms.
 template <int GD>
 GRNS_D int group_scale2pow_words(const DevCtx *c, const Group &g, int xi, unsigned D, bool &replay_ok) {
     const bool act = g.gl < g.L;
+    if constexpr (GD == 64) D = (unsigned)__builtin_amdgcn_readfirstlane((int)D);
     const int m = act ? c->m[g.gl] : 1;
     const double dinv = act ? c->dinv[g.gl] : 1.0;
     const int w = act ? c->w[g.gl] : 0;
+    const unsigned minv = act ? c->minv[g.gl] : 0u;
+    const unsigned fh = act ? c->wf_hi[g.gl] : 0u, fl = act ? c->wf_lo[g.gl] : 0u;
+    const unsigned yt = act ? c->rec_t[g.gl] : 0u, ylim = act ? c->rec_lim[g.gl] : 0u;
+    const bool fast = c->odd_moduli != 0;
     const unsigned X = group_words<GD>(c, g, xi);
+    const unsigned dig0 = digit30<GD>(g, X, g.gl), dig1 = digit30<GD>(g, X, g.gl + GD);
     const int xbits = 32 * wlen<GD>(g, X);
     const unsigned t = D / THRESH, dr = D % THRESH;
     const unsigned steps = t + (dr ? 1u : 0u);
-    int y = act ? xi : 0;  // lanes past n keep 0 throughout (m = 1, w = 0, inverses 0)
-    bool bad = false;
-    // (2^j)^-1 mod m for the full steps (j = THRESH) and the last one (j = dr), loaded once
-    const int inv_full = act && t ? c->pow2_inv[THRESH - 1][g.gl] : 0;
-    const int inv_last = act && dr ? c->pow2_inv[dr - 1][g.gl] : 0;
-    for (unsigned st = 0; st < steps; st++) {
-        const long long b = (long long)st * THRESH;
-        if (b >= xbits && group_all(g, !act || y == 0)) break;  // every later step maps 0 to 0
-        const int j = (st < t) ? THRESH : (int)dr;
-        unsigned r = 0;  // bits [b, b + j) of x
-        if (b < xbits) {
-            const int w0 = (int)(b >> 5), sh = (int)(b & 31);
-            const unsigned lo = gword<GD>(g, X, w0);
-            const unsigned hi = (sh && w0 + 1 < GD) ? gword<GD>(g, X, w0 + 1) : 0u;
-            r = (sh ? (lo >> sh) | (hi << (32 - sh)) : lo) & ((1u << j) - 1u);
+    int y = act ? xi : 0;  // lanes past n take no part (m = 1, w = 0, inverses 0)
+    bool bad = false, canon = true;
+    const unsigned long long lanes = __ballot(act) & group_mask_bits(g);
+    // steps with j = THRESH whose digit is in dig0: the tight loop
+    const unsigned tight = !fast ? 0u : (t < (unsigned)GD ? t : (unsigned)GD);
+    const unsigned minv30 = minv << (32 - THRESH);
+    unsigned st = 0;
+    while (st < steps) {
+        if (canon) {
+            for (; st < tight; st++) {
+                const int d = y - (int)gword<GD>(g, dig0, (int)st);
+                const unsigned y1 = (unsigned)(d >> THRESH) + (unsigned)m - __umulhi((unsigned)d * minv30, (unsigned)m);
+                const unsigned f = fh * (unsigned)y + __umulhi(fl, (unsigned)y);
+                if (scale_edges(y1 - yt, ylim, f) & lanes) break;
+                y = (int)y1;
+            }
+            if (st >= steps) break;
         }
-        const int cc = mulmod_recip(y, w, m, dinv);
-        bad |= (unsigned)cc >= (unsigned)m;
-        // rm = r % m and mult = (y - rm + m) % m as rem_trunc forms them: r < 2^30 and
-        // |y - rm + m| < 2^32 have exact doubles, formed from 32-bit pieces
-        const int rm = (int)rem_trunc_d((long long)r, (double)r, m, dinv);
-        const int mult = (int)rem_trunc_d((long long)y + (m - rm), (double)y + (double)(m - rm), m, dinv);
-        const int inv = st < t ? inv_full : inv_last;
-        const int qi = (int)(((double)mult * (double)inv) * dinv);
-        const long long v = (long long)mult * inv - (long long)qi * m;
-        bad |= v < -2147483648ll || v > 2147483647ll;
-        y = (int)v;
+        const int j = (st < t) ? THRESH : (int)dr;
+        unsigned r = st < (unsigned)GD       ? gword<GD>(g, dig0, (int)st)
+                     : st < 2u * (unsigned)GD ? gword<GD>(g, dig1, (int)st - GD)
+                                              : 0u;  // bits [30 st, 30 st + j) of x
+        r &= (1u << j) - 1u;
+        if (fast && canon && st >= tight) {
+            const int d = y - (int)r;
+            const unsigned v = (unsigned)(d >> j) - __umulhi(((unsigned)d * minv) << (32 - j), (unsigned)m);
+            const unsigned y1 = v + (unsigned)m < v ? v + (unsigned)m : v;  // v in [-m, m / 2]
+            const unsigned f = fh * (unsigned)y + __umulhi(fl, (unsigned)y);
+            if (!(scale_edges(y1 - yt, ylim, f) & lanes)) {
+                y = (int)y1;
+                st++;
+                continue;
+            }
+        }
+        // every later step maps 0 to 0
+        if ((long long)st * THRESH >= xbits && group_all(g, !act || y == 0)) break;
+        y = scale_step_reference(y, r, w, act ? c->pow2_inv[j - 1][g.gl] : 0, m, dinv, bad);
+        canon = group_all(g, !act || (unsigned)y < (unsigned)m);
+        st++;
     }
     replay_ok = !group_any(g, bad);
     return y;

@@ -109,6 +109,16 @@ grns_status build_constants(grns_ctx *c, const int *moduli, int n) {
             h.slo[i] = (shi - sh) + srem / (double)moduli[i];
         }
         h.c32[i] = (int)((1ull << 32) % (unsigned long long)m);
+        unsigned inv2 = (unsigned)m;  // m^-1 mod 2^3, then Newton steps doubling the bits (odd m)
+        for (int k = 0; k < 4; k++) inv2 *= 2u - (unsigned)m * inv2;
+        h.minv[i] = inv2;
+        const unsigned long long wf = (unsigned long long)((((unsigned __int128)(unsigned)h.w[i]) << 64) / (unsigned)m);
+        h.wf_hi[i] = (unsigned)(wf >> 32);
+        h.wf_lo[i] = (unsigned)wf;
+        // a reciprocal product below 2^31 m_i has a quotient within 3 2^-53 m_i of the true one, so
+        // it is canonical when the residue is at least 3 2^-53 m_i^2 from 0 and from m_i
+        h.rec_t[i] = (unsigned)(((unsigned long long)m * (unsigned long long)m) >> 51) + 2u;
+        h.rec_lim[i] = (unsigned)m > 2u * h.rec_t[i] ? (unsigned)m - 2u * h.rec_t[i] : 0u;
     }
     for (int t = 0; t < THRESH; t++) {
         unsigned long long mask = (1ull << (t + 1)) - 1;
@@ -137,6 +147,8 @@ grns_status build_constants(grns_ctx *c, const int *moduli, int n) {
     h.mr_lim = std::nextafter(1.0 / (double)moduli[n - 1], 2.0);
     h.m_min = moduli[0];
     for (int i = 1; i < n; i++) h.m_min = moduli[i] < h.m_min ? moduli[i] : h.m_min;
+    h.odd_moduli = 1;
+    for (int i = 0; i < n; i++) h.odd_moduli &= moduli[i] & 1;
     h.big_moduli = 1;
     for (int i = 0; i < n; i++) h.big_moduli &= (moduli[i] >= (1 << 22));
     // RNS_EVAL_UNIT / INV_UNIT: M rounded down to 53 bits, then 1/Md and 1 - 1/Md rounded up and
