@@ -6,6 +6,7 @@
 
 #include "../../include/grns.h"
 #include "grns_kernels.hpp"
+#include "grns_matrix.hpp"
 
 struct grns_ctx {
     int device = 0;
@@ -17,6 +18,8 @@ struct grns_ctx {
     int *d_mrc = nullptr;
     int *d_mrc_acc = nullptr;     // DevCtx::mrc_acc
     int *d_status = nullptr;
+    unsigned char *d_mat = nullptr;  // tables of the matrix-core conversions (sets of up to 64 moduli)
+    grns::MatTab mat = {};           // their device addresses
     unsigned *d_crt = nullptr;      // DevCtx::crt_words
     int max_blocks = 2048;         // arg-max stage-1 grid, from the occupancy query (max_grid_for)
     int max_blocks_occ = 2048;     // the same as set at context creation (test hooks restore it)
@@ -68,5 +71,16 @@ inline int words_group(const grns_ctx *c) {
     return G <= 64 ? G : 0;
 }
 
-namespace grns {
-}  // namespace grns
+// Conversions of at least this many numbers run on the matrix cores, shorter ones with a wave group per
+// number.  A wave of the matrix form takes 32 or 64 numbers and first loads its tables, so short
+// calls leave the chip idle: with 64 moduli 8192 numbers take 11-14 us by groups and 11-15 us on the
+// matrix cores, 16384 take 21-25 us and 11-15 us; with 32 moduli both take 8.5-9.5 us at 8192
+// numbers, and 16384 take 10-12 us and 8.5-9.5 us.
+inline size_t matrix_min(const grns_ctx *c) { return c->n > 32 ? 16384 : 8192; }
+
+// Matrix-core conversions (grns_matrix.hip): tables at context creation, and the launches.
+grns_status matrix_tables_create(grns_ctx *c);
+grns_status matrix_to_binary(grns_ctx *c, const int *x, long long smod, long long snum, size_t count, unsigned *w,
+                             long long wst, long long wsn, hipStream_t s);
+grns_status matrix_from_binary(grns_ctx *c, const unsigned *w, long long wst, long long wsn, int nwords, const int *sign,
+                               size_t count, int *x, long long smod, long long snum, hipStream_t s);

@@ -1743,8 +1743,20 @@ __global__ __launch_bounds__(BLOCK) void k_from_binary(const DevCtx *__restrict_
     }
 }
 
-// rns_to_binary (src/rnsbase.cuh:277-287): each residue reduced as the reference's mpz_mul_ui
-// sees it (an int cast to unsigned long: x_i + 2^64 when negative), then the words of the CRT value.
+// Residue i as the reference's mpz_mul_ui sees it (an int cast to unsigned long: x_i + 2^64 when
+// negative), mod m_i.
+GRNS_D int unsigned_long_residue(const DevCtx *c, int xi, int i) {
+    const int m = c->m[i];
+    const double dinv = c->dinv[i];
+    long long r = rem_trunc((long long)xi, m, dinv);
+    if (xi < 0) {
+        const long long c32 = c->c32[i], p64 = rem_trunc(c32 * c32, m, dinv);  // 2^64 mod m
+        r = rem_trunc(r + p64 + m, m, dinv);
+    }
+    return (int)r;
+}
+
+// rns_to_binary (src/rnsbase.cuh:277-287): the words of the CRT value of each number.
 template <int GD>
 __global__ __launch_bounds__(BLOCK) void k_to_binary(const DevCtx *__restrict__ c, const int *__restrict__ x,
                                                      long long smod, long long snum, long long count,
@@ -1754,21 +1766,11 @@ __global__ __launch_bounds__(BLOCK) void k_to_binary(const DevCtx *__restrict__ 
     const long long wave = ((long long)xcd_block() * BLOCK + threadIdx.x) >> 6;
     const long long nwaves = ((long long)gridDim.x * BLOCK) >> 6;
     const bool act = g.gl < g.L;
-    const int m = act ? c->m[g.gl] : 1;
-    const double dinv = act ? c->dinv[g.gl] : 1.0;
-    const long long c32 = act ? c->c32[g.gl] : 0;
-    const long long p64 = act ? rem_trunc(c32 * c32, m, dinv) : 0;  // 2^64 mod m
     const int W = c->words - 1;
     for (long long j0 = wave * P; j0 < count; j0 += nwaves * P) {
         const long long j = j0 + (threadIdx.x & 63) / GD;
         if (j >= count) continue;
-        int xi = 0;
-        if (act) {
-            const long long v = x[j * snum + (long long)g.gl * smod];
-            long long r = rem_trunc(v, m, dinv);
-            if (v < 0) r = rem_trunc(r + p64 + m, m, dinv);
-            xi = (int)r;
-        }
+        const int xi = act ? unsigned_long_residue(c, x[j * snum + (long long)g.gl * smod], g.gl) : 0;
         const unsigned X = group_words<GD>(c, g, xi);
         if (g.gl < W) w[j * wsn + (long long)g.gl * wst] = X;
     }

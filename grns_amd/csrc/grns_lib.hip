@@ -459,6 +459,7 @@ grns_status grns_ctx_create(const int *moduli, int n, int device, grns_ctx **out
         hipMemcpy(c->d_mrc_acc, c->mrc_acc.data(), sizeof(int) * c->mrc_acc.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d, &c->h, sizeof(DevCtx), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(c->d_status, 0, sizeof(int)) != hipSuccess ||
+        matrix_tables_create(c) != GRNS_OK ||
         hipDeviceSynchronize() != hipSuccess) {  // tables and status in place before any stream's kernels
         grns_ctx_destroy(c);
         return GRNS_ERR_HIP;
@@ -482,6 +483,7 @@ grns_status grns_ctx_destroy(grns_ctx *c) {
         if (c->d_mrc) (void)hipFree(c->d_mrc);
         if (c->d_mrc_acc) (void)hipFree(c->d_mrc_acc);
         if (c->d_status) (void)hipFree(c->d_status);
+        if (c->d_mat) (void)hipFree(c->d_mat);
         for (auto &q : c->queues) {
             (void)hipFree(q.items);
             (void)hipFree(q.ctr);
@@ -735,6 +737,7 @@ grns_status grns_from_binary(grns_ctx *c, const unsigned *w, long long wst, long
     if (count == 0) return GRNS_OK;
     if (c->n > 64) return GRNS_ERR_UNSUPPORTED;
     DeviceGuard guard(c->device);
+    if (count >= matrix_min(c)) return matrix_from_binary(c, w, wst, wsn, nwords, sign, count, x, smod, snum, S(stream));
     const int G = groups_for(c->n);
     dim3 grid((unsigned)grid_groups(count, G)), blk(BLOCK);
     const long long cnt = (long long)count;
@@ -758,6 +761,7 @@ grns_status grns_to_binary(grns_ctx *c, const int *x, long long smod, long long 
     const int GW = words_group(c);
     if (c->n > 64 || !GW) return GRNS_ERR_UNSUPPORTED;
     DeviceGuard guard(c->device);
+    if (count >= matrix_min(c)) return matrix_to_binary(c, x, smod, snum, count, w, wst, wsn, S(stream));
     dim3 grid((unsigned)grid_groups(count, GW)), blk(BLOCK);
     const long long cnt = (long long)count;
     switch (GW) {
