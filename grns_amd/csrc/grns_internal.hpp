@@ -84,3 +84,13 @@ grns_status matrix_to_binary(grns_ctx *c, const int *x, long long smod, long lon
                              long long wst, long long wsn, hipStream_t s);
 grns_status matrix_from_binary(grns_ctx *c, const unsigned *w, long long wst, long long wsn, int nwords, const int *sign,
                                size_t count, int *x, long long smod, long long snum, hipStream_t s);
+// Divisions of at least this many pairs take a lane per pair (grns_divide.hip), shorter ones a wave
+// group per pair: 64 pairs to a wave leave the chip idle below.  Divisors of uniform length: 16384 pairs
+// of 8, 16, 32, 64 moduli take 19, 36, 54, 93 us by groups and 18, 23, 38, 82 us by lanes; the groups'
+// time falls with the quotient's length, to 16, 21, 26, 45 us for divisors as long as the dividend
+// (16, 19, 30, 57 us by lanes), hence the higher line above 16 moduli.
+inline size_t div_lanes_min(const grns_ctx *c) { return c->n > 16 ? 32768 : 16384; }
+
+// Lane-per-pair division (grns_divide.hip): pairs it does not take go to the rare queue.
+grns_status matrix_div(grns_ctx *c, const int *x, const int *d, long long smod, long long snum, size_t count, int *q,
+                       int *r, const grns::RareQ &rq, hipStream_t s);

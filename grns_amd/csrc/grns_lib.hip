@@ -677,7 +677,10 @@ grns_status grns_div(grns_ctx *c, const int *x, const int *d, long long smod, lo
         grns_status qs = rare_queue(c, stream, rq);
         if (qs != GRNS_OK) return qs;
         dim3 gw((unsigned)grid_groups(count, GW)), rg((unsigned)rare_grid(count));
-        switch (GW) {
+        if (count >= div_lanes_min(c)) {
+            qs = matrix_div(c, x, d, smod, snum, count, q, r, rq, S(stream));
+            if (qs != GRNS_OK) return qs;
+        } else switch (GW) {
             case 2: hipLaunchKernelGGL((k_div_words<2>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
             case 4: hipLaunchKernelGGL((k_div_words<4>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
             case 8: hipLaunchKernelGGL((k_div_words<8>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;

@@ -70,13 +70,15 @@ grns_status matrix_tables_create(grns_ctx *c) {
     const int n = c->n;
     if (n > 64) return GRNS_OK;
     const int NP = n <= 8 ? 8 : n <= 16 ? 16 : n <= 32 ? 32 : 64;
-    const int T8 = NP / 8, WW = c->h.words;
+    const int T8 = NP / 8, DT = ((31 * NP + 27) / 28 + 7) / 8, WW = c->h.words;
     Layout L;
     const size_t rec_at = L.take(sizeof(ModRec) * NP);
     const size_t crt8_at = L.take((size_t)T8 * T8 * 1024), crt8i_at = L.take((size_t)T8 * 32 * 4);
     const size_t m8_at = L.take((size_t)NP * 4), m32_at = L.take((size_t)NP * 4);
     const size_t res8_at = L.take((size_t)T8 * T8 * 1024), res8i_at = L.take((size_t)T8 * 32 * 4);
     const size_t fold_at = L.take((size_t)NP * 4);
+    const size_t crt7_at = L.take((size_t)DT * T8 * 1024), crt7i_at = L.take((size_t)DT * 32 * 4);
+    const size_t m28_at = L.take((size_t)DT * 8 * 4), res7_at = L.take((size_t)T8 * DT * 1024);
     std::vector<unsigned char> host(L.size, 0);
 
     ModRec *rec = reinterpret_cast<ModRec *>(host.data() + rec_at);
@@ -87,29 +89,39 @@ grns_status matrix_tables_create(grns_ctx *c) {
             rec[i].m = (unsigned)c->h.m[i];
             rec[i].w = (unsigned)c->h.w[i];
             rec[i].wf = c->h.wf_hi[i];
+            rec[i].keeps_m = (double)c->h.m[i] * c->h.dinv[i] < 1.0;
             rec[i].dinv = c->h.dinv[i];
             rec[i].hdinv = 0.5 * c->h.dinv[i];
         }
     }
-    // digits of 2^(8 a) M / m_i, one vector per (i, a), and of M
+    // digits of 2^(8 a) M / m_i in base 2^bits, one vector per K index 4 i + a; row (mt, q, h, b) is
+    // column b of digit 4 tiles h + 4 mt + q
     std::vector<std::vector<int>> crt((size_t)4 * NP);
-    for (int i = 0; i < n; i++)
-        for (int a = 0; a < 4; a++) {
-            std::vector<unsigned> v(WW + 1, 0u);
-            for (int k = 0; k < WW; k++) {
-                const unsigned long long t = (unsigned long long)c->crt[(size_t)i * WW + k] << (8 * a);
-                v[k] |= (unsigned)t;
-                v[k + 1] = (unsigned)(t >> 32);
+    auto crt_digits_of = [&](int bits, int tiles, bool balanced) {
+        for (int i = 0; i < n; i++)
+            for (int a = 0; a < 4; a++) {
+                std::vector<unsigned> v(WW + 1, 0u);
+                for (int k = 0; k < WW; k++) {
+                    const unsigned long long t = (unsigned long long)c->crt[(size_t)i * WW + k] << (8 * a);
+                    v[k] |= (unsigned)t;
+                    v[k + 1] = (unsigned)(t >> 32);
+                }
+                split_digits(v, bits, 32 * tiles, balanced, crt[(size_t)4 * i + a]);
             }
-            split_digits(v, 8, 4 * NP, true, crt[(size_t)4 * i + a]);
-        }
-    auto crt_value = [&](int mt, int row, int kk) {
-        const std::vector<int> &d = crt[kk];  // kk = 4 i + a
-        const int q = row / 8, h = (row % 8) / 4, b = row % 4;
-        return d.empty() ? 0 : d[4 * (4 * T8 * h + 4 * mt + q) + b];
     };
-    fill_fragments(reinterpret_cast<signed char *>(host.data() + crt8_at), T8, T8, crt_value);
-    fill_init(reinterpret_cast<int *>(host.data() + crt8i_at), T8, T8, crt_value);
+    auto crt_value = [&](int tiles) {
+        return [&crt, tiles](int mt, int row, int kk) {
+            const std::vector<int> &d = crt[kk];
+            const int q = row / 8, h = (row % 8) / 4, b = row % 4;
+            return d.empty() ? 0 : d[4 * (4 * tiles * h + 4 * mt + q) + b];
+        };
+    };
+    crt_digits_of(8, T8, true);
+    fill_fragments(reinterpret_cast<signed char *>(host.data() + crt8_at), T8, T8, crt_value(T8));
+    fill_init(reinterpret_cast<int *>(host.data() + crt8i_at), T8, T8, crt_value(T8));
+    crt_digits_of(7, DT, false);
+    fill_fragments(reinterpret_cast<signed char *>(host.data() + crt7_at), DT, T8, crt_value(DT));
+    fill_init(reinterpret_cast<int *>(host.data() + crt7i_at), DT, T8, crt_value(DT));
     {
         int *m8 = reinterpret_cast<int *>(host.data() + m8_at);
         unsigned *m32 = reinterpret_cast<unsigned *>(host.data() + m32_at);
@@ -120,25 +132,36 @@ grns_status matrix_tables_create(grns_ctx *c) {
             m8[k] = (int)(unsigned)v;
             carry = v >= 0x80000000ull ? 1u : 0u;  // the digit is v - 2^32
         }
+        std::vector<int> d28;
+        split_digits(std::vector<unsigned>(c->crt.begin() + (size_t)n * WW, c->crt.end()), 28, 8 * DT, false, d28);
+        std::memcpy(host.data() + m28_at, d28.data(), d28.size() * 4);
     }
-    // bytes of 2^(8 c) mod m_i, centred
-    std::vector<std::vector<int>> pw(NP, std::vector<int>((size_t)4 * NP, 0));
-    for (int i = 0; i < n; i++) {
-        const long long m = c->h.m[i];
-        long long p = 1 % m;
-        for (int k = 0; k < 4 * NP; k++) {
-            pw[i][k] = (int)(p > m / 2 ? p - m : p);
-            p = p * 256 % m;
+    // bytes of 2^(bits c) mod m_i, centred; K index c is byte (or 7-bit piece) c of the integer, row
+    // (mt, q, h, b) byte b of modulus 8 mt + 4 h + q
+    std::vector<std::vector<int>> pw(NP);
+    auto powers = [&](int bits, int cols) {
+        for (int i = 0; i < NP; i++) {
+            pw[i].assign(cols, 0);
+            if (i >= n) continue;
+            const long long m = c->h.m[i];
+            long long p = 1 % m;
+            for (int k = 0; k < cols; k++) {
+                pw[i][k] = (int)(p > m / 2 ? p - m : p);
+                p = (p << bits) % m;
+            }
+            if (bits == 8) reinterpret_cast<unsigned *>(host.data() + fold_at)[i] = (unsigned)p;
         }
-        reinterpret_cast<unsigned *>(host.data() + fold_at)[i] = (unsigned)p;
-    }
+    };
     auto res_value = [&](int mt, int row, int kk) {
         const int q = row / 8, h = (row % 8) / 4, b = row % 4;
         const unsigned t = (unsigned)pw[8 * mt + 4 * h + q][kk] + 0x80808080u;
         return (int)((t >> (8 * b)) & 255u) - 128;
     };
+    powers(8, 4 * NP);
     fill_fragments(reinterpret_cast<signed char *>(host.data() + res8_at), T8, T8, res_value);
     fill_init(reinterpret_cast<int *>(host.data() + res8i_at), T8, T8, res_value);
+    powers(7, 32 * DT);
+    fill_fragments(reinterpret_cast<signed char *>(host.data() + res7_at), T8, DT, res_value);
 
     if (hipMalloc(&c->d_mat, L.size) != hipSuccess) return GRNS_ERR_OOM;
     if (hipMemcpy(c->d_mat, host.data(), L.size, hipMemcpyHostToDevice) != hipSuccess) return GRNS_ERR_HIP;
@@ -151,6 +174,10 @@ grns_status matrix_tables_create(grns_ctx *c) {
     c->mat.res8 = reinterpret_cast<const v4i *>(d + res8_at);
     c->mat.res8_init = reinterpret_cast<const int *>(d + res8i_at);
     c->mat.fold = reinterpret_cast<const unsigned *>(d + fold_at);
+    c->mat.crt7 = reinterpret_cast<const v4i *>(d + crt7_at);
+    c->mat.crt7_init = reinterpret_cast<const int *>(d + crt7i_at);
+    c->mat.m28 = reinterpret_cast<const int *>(d + m28_at);
+    c->mat.res7 = reinterpret_cast<const v4i *>(d + res7_at);
     return GRNS_OK;
 }
 

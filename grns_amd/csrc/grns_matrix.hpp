@@ -23,7 +23,8 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // Per-modulus constants of the conversions.  Records past the set's n (up to the padded count) have
 // m = 2^32 - 1 and zeros: any residue is canonical and its term is 0.
 struct ModRec {
-    unsigned m, w, wf, pad;  // wf = floor(2^32 w / m)
+    unsigned m, w, wf;  // wf = floor(2^32 w / m)
+    unsigned keeps_m;   // RN(m RN(1 / m)) < 1: a reciprocal addition leaves m where the sum is m
     double dinv, hdinv;      // RN(1 / m) and half of it
 };
 
@@ -34,6 +35,9 @@ struct Mat {
     static constexpr int RT = NP / 8;               // row tiles of residues: 8 moduli of 4 bytes
     static constexpr int WT = NP / 8;               // row tiles of 32-bit words: 8 words of 4 bytes
     static constexpr int KW = NP / 8;               // K steps over words
+    static constexpr int ND = (31 * NP + 27) / 28;  // 28-bit digits of M < 2^(31 NP); the top one stays below 2^27
+    static constexpr int DT = (ND + 7) / 8;         // row tiles of digits: 8 digits of 4 columns of 7 bits
+    static constexpr int KD = DT;                   // K steps over digits
 };
 
 // Device tables of one context (fragments in the order the wave loads them: 64 lanes x 16 bytes).
@@ -46,6 +50,10 @@ struct MatTab {
     const v4i *res8;       // [RT][KW][64]: bytes in [-128, 127] of 2^(8 c) mod m_i, centred
     const int *res8_init;  // [RT][2][16]
     const unsigned *fold;  // [NP]: 2^(32 NP) mod m_i
+    const v4i *crt7;       // [DT][KR][64]: digits of 2^(8 a) M / m_i, base 2^7
+    const int *crt7_init;  // [DT][2][16]
+    const int *m28;        // [2][4 DT]: M in base 2^28
+    const v4i *res7;       // [RT][KD][64]: bytes in [-128, 127] of 2^(7 c) mod m_i, centred
 };
 
 // s_i = x_i w_i mod m_i, plus m_i at times: below 2 m_i < 2^32 for any 32-bit x_i.
@@ -176,6 +184,7 @@ template <int CB>
 GRNS_D int digits_join(const DigitColumn &col, int H, int h, int carry) {
     const int c0 = other_half(carry);
     int c = h ? c0 : 0;
+#pragma unroll 1
     for (int k = 0; k < H && __any(c != 0); k++) {
         unsigned &d = col.at(h * H + k);
         const long long v = (long long)d + c;
@@ -186,50 +195,75 @@ GRNS_D int digits_join(const DigitColumn &col, int H, int h, int carry) {
     return h ? top : o;
 }
 
-// The value sum_i s_i M_i - k M of the lane pair's number, as digits in base 2^(4 CB) in LDS: lane half h
-// writes digits 4 MT h + 0 .. 4 MT - 1.  The column sums of one row tile are four digits of the half:
-// with |C| < 2^23 the sums of two columns fit 32 bits.  MU row tiles at a time, so that the matrix
-// core has independent sums to work on.  The loop over row tiles is rolled: unrolled, the code of
-// a pass did not fit the instruction cache.
-template <int NP, int CB, int MT, int MU>
+// The values sum_i s_i M_i - k M of the lane pair's numbers (one per tile), as digits in base 2^(4 CB)
+// in LDS: lane half h writes digits 4 MT h + 0 .. 4 MT - 1 of col[t].  The column sums of one row tile
+// are four digits of the half: with |C| < 2^23 the sums of two columns fit 32 bits.  MU row tiles at a
+// time, so that the matrix core has independent sums to work on.  The loop over row tiles is rolled:
+// unrolled, the code of a pass did not fit the instruction cache.
+template <int NP, int CB, int MT, int MU, int T>
 GRNS_D void crt_digits(const v4i *frags, const int *init, const int *mdig, const unsigned *mpos,
-                       const v4i (&B)[Mat<NP>::KR], int k, int lane, const DigitColumn &col) {
+                       const v4i (&B)[T][Mat<NP>::KR], const int (&k)[T], int lane, const DigitColumn (&col)[T]) {
     constexpr int KR = Mat<NP>::KR, H = 4 * MT;
     const int h = lane >> 5;
-    long long carry = 0;
+    long long carry[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) carry[t] = 0;
+    v4i a[MU][KR];
+    auto load_rows = [&](int m0) {
+#pragma unroll
+        for (int u = 0; u < MU; u++)
+#pragma unroll
+            for (int ks = 0; ks < KR; ks++) a[u][ks] = frags[((m0 + u) * KR + ks) * 64 + lane];
+    };
+    load_rows(0);
 #pragma unroll 1
     for (int m0 = 0; m0 < MT; m0 += MU) {
-        v16i acc[MU];
+        v16i acc[MU][T];
 #pragma unroll
-        for (int u = 0; u < MU; u++) acc[u] = load_init(init + ((m0 + u) * 2 + h) * 16);
+        for (int u = 0; u < MU; u++) {
+            acc[u][0] = load_init(init + ((m0 + u) * 2 + h) * 16);
+#pragma unroll
+            for (int t = 1; t < T; t++) acc[u][t] = acc[u][0];
+        }
 #pragma unroll
         for (int ks = 0; ks < KR; ks++)
 #pragma unroll
             for (int u = 0; u < MU; u++)
-                acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(frags[((m0 + u) * KR + ks) * 64 + lane], B[ks], acc[u], 0,
-                                                               0, 0);
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    acc[u][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][ks], B[t][ks], acc[u][t], 0, 0, 0);
+        sched_stop();
+        load_rows(m0 + MU < MT ? m0 + MU : 0);  // the next rows arrive while the digits are formed
+        sched_stop();
 #pragma unroll
         for (int u = 0; u < MU; u++) {
             const v4i mw = *reinterpret_cast<const v4i *>(mdig + h * H + 4 * (m0 + u));
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int lo = acc[u][4 * q] + (acc[u][4 * q + 1] << CB);
-                const int hi = acc[u][4 * q + 2] + (acc[u][4 * q + 3] << CB);
-                const long long v = carry + (long long)hi * (1 << (2 * CB)) + lo - (long long)k * mw[q];
-                col.at(h * H + 4 * (m0 + u) + q) = (unsigned)v & (unsigned)((1ull << (4 * CB)) - 1);
-                carry = v >> (4 * CB);
+            for (int t = 0; t < T; t++) {
+                const v16i &C = acc[u][t];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int lo = C[4 * q] + (C[4 * q + 1] << CB), hi = C[4 * q + 2] + (C[4 * q + 3] << CB);
+                    const long long v = carry[t] + (long long)hi * (1 << (2 * CB)) + lo - (long long)k[t] * mw[q];
+                    col[t].at(h * H + 4 * (m0 + u) + q) = (unsigned)v & (unsigned)((1ull << (4 * CB)) - 1);
+                    carry[t] = v >> (4 * CB);
+                }
             }
         }
     }
-    const bool neg = digits_join<CB>(col, H, h, (int)carry) < 0;
-    if (__any(neg)) {  // within 2^-30 M of M: M is added back
-        long long c = 0;
-        for (int d = h * H; d < h * H + H; d++) {
-            const long long v = (long long)col.at(d) + (neg ? (long long)mpos[d] : 0) + c;
-            col.at(d) = (unsigned)v & (unsigned)((1ull << (4 * CB)) - 1);
-            c = v >> (4 * CB);
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        const bool neg = digits_join<CB>(col[t], H, h, (int)carry[t]) < 0;
+        if (__any(neg)) {  // within 2^-30 M of M: M is added back
+            long long c = 0;
+#pragma unroll 1
+            for (int d = h * H; d < h * H + H; d++) {
+                const long long v = (long long)col[t].at(d) + (neg ? (long long)mpos[d] : 0) + c;
+                col[t].at(d) = (unsigned)v & (unsigned)((1ull << (4 * CB)) - 1);
+                c = v >> (4 * CB);
+            }
+            (void)digits_join<CB>(col[t], H, h, (int)c);
         }
-        (void)digits_join<CB>(col, H, h, (int)c);
     }
 }
 
@@ -262,7 +296,7 @@ __global__ __launch_bounds__(to_binary_block(NP), 2) void k_to_binary_mat(const 
     const bool packed = wst == 1 && wsn == nw && ((uintptr_t)w & 15) == 0;
     const bool quad = quads(x, smod, snum);
     unsigned *st = stage[threadIdx.x >> 6];
-    const DigitColumn col{st + (lane & 31) * nw, st + 32 * nw + (lane & 31) * (NP - nw) - nw, 1, nw};
+    const DigitColumn col[1] = {{st + (lane & 31) * nw, st + 32 * nw + (lane & 31) * (NP - nw) - nw, 1, nw}};
     for (long long tile = wave; tile < tiles; tile += nwaves) {
         const long long j0 = tile * 32, j = j0 + (lane & 31);
         const int *p[1] = {x + (j < count ? j : count - 1) * snum};
@@ -271,7 +305,7 @@ __global__ __launch_bounds__(to_binary_block(NP), 2) void k_to_binary_mat(const 
         LaneAny bad[1];
         load_residues<NP, 1>(p, smod, quad, n, h, B);
         crt_operand<NP, 1>(rec, h, B, k, bad);
-        crt_digits<NP, 8, WT, WT >= 2 ? 2 : 1>(table, init, mdig, tab.m32, B[0], k[0], lane, col);
+        crt_digits<NP, 8, WT, WT >= 2 ? 2 : 1, 1>(table, init, mdig, tab.m32, B, k, lane, col);
         wave_lds_fence();
         const int valid = (int)(count - j0 < 32 ? count - j0 : 32);
         if (packed) {
