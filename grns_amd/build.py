@@ -17,8 +17,9 @@ LIB = os.path.join(HERE, "libgrns_hip.so")
 WORKLOAD_LIB = os.path.join(HERE, "libgrns_workload.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["grns_lib.hip", "grns_batch.hip", "grns_matrix.hip", "grns_divide.hip"]
-HEADERS = ["grns_device.hpp", "grns_kernels.hpp", "grns_matrix.hpp", "grns_divide.hpp", "grns_internal.hpp"]
+SOURCES = ["grns_lib.hip", "grns_batch.hip", "grns_matrix.hip", "grns_divide.hip", "grns_scale.hip"]
+HEADERS = ["grns_device.hpp", "grns_kernels.hpp", "grns_matrix.hpp", "grns_divide.hpp", "grns_scale.hpp",
+           "grns_internal.hpp"]
 
 FLAGS = [
     "--offload-arch=gfx950",

@@ -183,22 +183,15 @@ __global__ __launch_bounds__(BLOCK) void k_batch_div(const DevCtx *__restrict__ 
     });
 }
 
-// Scaling (group of GD lanes per number): the replay, or the reference steps for the numbers it
-// does not take.
+// Scaling (group of GD lanes per number).
 template <int GD>
 __global__ __launch_bounds__(BLOCK) void k_batch_scale(const DevCtx *__restrict__ c,
                                                        const BatchTask *__restrict__ tasks, int ntasks,
                                                        long long total, int tile, unsigned long long *counter) {
     for_group_tiles(c, GD, tasks, ntasks, total, tile, counter, [&](const BatchTask &T, const Group &g, long long j) {
-        const bool act = g.gl < g.L;
         const long long oa = j * T.asn + (long long)g.gl * T.asm_;
-        const int xi = act ? T.a[oa] : 0;
-        const unsigned Dj = T.D[j];
-        bool ok = false;
-        int v = 0;
-        if (group_all(g, !act || (unsigned)xi < (unsigned)c->m[g.gl])) v = group_scale2pow_words<GD>(c, g, xi, Dj, ok);
-        if (!ok) v = group_scale2pow(c, g, xi, Dj);
-        if (act) reinterpret_cast<int *>(T.o0)[oa] = v;
+        const int v = group_scale2pow_words<GD>(c, g, g.gl < g.L ? T.a[oa] : 0, T.D[j]);
+        if (g.gl < g.L) reinterpret_cast<int *>(T.o0)[oa] = v;
     });
 }
 

@@ -626,11 +626,6 @@ GRNS_D double group_psum(const Group &g, double v) {
     return v;
 }
 
-GRNS_D long long group_sum_ll(const Group &g, long long v) {
-    for (int h = 1; h < g.G; h <<= 1) v += __shfl_xor(v, h, 64);
-    return v;
-}
-
 // ---------------------------------------------------------------- position certificates
 // Sign of the top mixed-radix digit of a canonical x (all the reference's ambiguity branch reads of
 // the conversion, src/rnseval.cuh:62-65) from its position, or -1 when the position leaves it
@@ -1131,117 +1126,6 @@ GRNS_D void group_div_words(const DevCtx *c, const Group &g, int xi, int di, int
         q = (qnz && qr == 0 && (double)m * dinv < 1.0) ? m : qr;
         r = psubmod(xi, mulmod3(qr, di, m, dinv), m, dinv);
     }
-}
-
-// One step of the replay below as the reference computes it, for any y it may hold: X_s mod 2^j is
-// r, inv is (2^j)^-1 mod m.  `bad`: c = y w is not canonical, or y' wraps int32.
-GRNS_D int scale_step_reference(int y, unsigned r, int w, int inv, int m, double dinv, bool &bad) {
-    const int cc = mulmod_recip(y, w, m, dinv);
-    bad |= (unsigned)cc >= (unsigned)m;
-    // rm = r % m and mult = (y - rm + m) % m as rem_trunc forms them: r < 2^30 and
-    // |y - rm + m| < 2^32 have exact doubles, formed from 32-bit pieces
-    const int rm = (int)rem_trunc_d((long long)r, (double)r, m, dinv);
-    const int mult = (int)rem_trunc_d((long long)y + (m - rm), (double)y + (double)(m - rm), m, dinv);
-    const int qi = (int)(((double)mult * (double)inv) * dinv);
-    const long long v = (long long)mult * inv - (long long)qi * m;
-    bad |= v < -2147483648ll || v > 2147483647ll;
-    return (int)v;
-}
-
-// Bits [30 l, 30 l + 30) of the group's value, l >= 0 the lane's own choice.
-template <int GD>
-GRNS_D unsigned digit30(const Group &g, unsigned X, int l) {
-    const int b = 30 * l, w0 = b >> 5, sh = b & 31;
-    unsigned lo = (unsigned)__shfl((int)X, g.base + (w0 < GD ? w0 : 0), 64);
-    unsigned hi = (unsigned)__shfl((int)X, g.base + (w0 + 1 < GD ? w0 + 1 : 0), 64);
-    lo = w0 < GD ? lo : 0u;
-    hi = w0 + 1 < GD ? hi : 0u;
-    return (unsigned)((((unsigned long long)hi << 32) | lo) >> sh) & 0x3fffffffu;
-}
-
-// The active lanes whose y' (yo = y' - rec_t) or fraction f of y w / m (32 bits, at most 2 below
-// the true one) is too near the edges: both limits keep a fraction 2^-20 from an integer.
-GRNS_D unsigned long long scale_edges(unsigned yo, unsigned ylim, unsigned f) {
-    return __builtin_amdgcn_uicmp(yo, ylim, 35) | __builtin_amdgcn_uicmp(f - 4100u, 0u - 8200u, 35);  // ICMP_UGE
-}
-
-// rns_scale2pow (src/rnsscal.cuh:93-119) replayed on the words of a canonical x.  Step s of the
-// reference maps its value X_s = floor(x / 2^(30 s)) to X_{s+1} = floor(X_s / 2^j): with its
-// residues y (as the reference holds them, possibly y + m or y - m) it forms c = y * w (for the
-// rank), X_s mod 2^j, multiple = (y - (X_s mod 2^j) mod m + m) % m and y' = multiple * (2^j)^-1,
-// the products by reciprocal reduction.  Whenever every c is canonical, the rank and the residue
-// X_s mod 2^j of the reference are consistent, so X_s mod 2^j is the word bits [30 s, 30 s + j)
-// of x, and y' follows from y exactly as the reference computes it.  A step whose c is not
-// canonical or whose y' wraps int32 (the reference then continues with another number) sets
-// `replay_ok` false and the caller runs the reference steps instead.
-//
-// A reciprocal product is canonical unless its fraction is within 2^-20.4 of an integer.  So a step
-// from canonical y first takes its y' by exact division, y' = (y - r) / 2^j mod m = (d - h m) / 2^j
-// with d = y - r and h = d m^-1 mod 2^j (two 32-bit multiplications: the low parts of d and h m are
-// equal, so the high parts alone give the quotient), and the fraction of y w / m to 32 bits (two
-// more): when every lane's y' and fraction keep their distance from the edges, the reference's
-// products are canonical and y' is its result.  Otherwise the step (one in about 10^4, and those
-// near the end of a small value) runs as the reference computes it; so does every step of a set
-// with an even modulus, which has no inverse of 2.  13 vector instructions per step instead of 64:
-// 2^20 numbers of 64 moduli with D uniform in [1, 1900] take 2.3 ms instead of 5.0 ms.
-template <int GD>
-GRNS_D int group_scale2pow_words(const DevCtx *c, const Group &g, int xi, unsigned D, bool &replay_ok) {
-    const bool act = g.gl < g.L;
-    if constexpr (GD == 64) D = (unsigned)__builtin_amdgcn_readfirstlane((int)D);
-    const int m = act ? c->m[g.gl] : 1;
-    const double dinv = act ? c->dinv[g.gl] : 1.0;
-    const int w = act ? c->w[g.gl] : 0;
-    const unsigned minv = act ? c->minv[g.gl] : 0u;
-    const unsigned fh = act ? c->wf_hi[g.gl] : 0u, fl = act ? c->wf_lo[g.gl] : 0u;
-    const unsigned yt = act ? c->rec_t[g.gl] : 0u, ylim = act ? c->rec_lim[g.gl] : 0u;
-    const bool fast = c->odd_moduli != 0;
-    const unsigned X = group_words<GD>(c, g, xi);
-    const unsigned dig0 = digit30<GD>(g, X, g.gl), dig1 = digit30<GD>(g, X, g.gl + GD);
-    const int xbits = 32 * wlen<GD>(g, X);
-    const unsigned t = D / THRESH, dr = D % THRESH;
-    const unsigned steps = t + (dr ? 1u : 0u);
-    int y = act ? xi : 0;  // lanes past n take no part (m = 1, w = 0, inverses 0)
-    bool bad = false, canon = true;
-    const unsigned long long lanes = __ballot(act) & group_mask_bits(g);
-    // steps with j = THRESH whose digit is in dig0: the tight loop
-    const unsigned tight = !fast ? 0u : (t < (unsigned)GD ? t : (unsigned)GD);
-    const unsigned minv30 = minv << (32 - THRESH);
-    unsigned st = 0;
-    while (st < steps) {
-        if (canon) {
-            for (; st < tight; st++) {
-                const int d = y - (int)gword<GD>(g, dig0, (int)st);
-                const unsigned y1 = (unsigned)(d >> THRESH) + (unsigned)m - __umulhi((unsigned)d * minv30, (unsigned)m);
-                const unsigned f = fh * (unsigned)y + __umulhi(fl, (unsigned)y);
-                if (scale_edges(y1 - yt, ylim, f) & lanes) break;
-                y = (int)y1;
-            }
-            if (st >= steps) break;
-        }
-        const int j = (st < t) ? THRESH : (int)dr;
-        unsigned r = st < (unsigned)GD       ? gword<GD>(g, dig0, (int)st)
-                     : st < 2u * (unsigned)GD ? gword<GD>(g, dig1, (int)st - GD)
-                                              : 0u;  // bits [30 st, 30 st + j) of x
-        r &= (1u << j) - 1u;
-        if (fast && canon && st >= tight) {
-            const int d = y - (int)r;
-            const unsigned v = (unsigned)(d >> j) - __umulhi(((unsigned)d * minv) << (32 - j), (unsigned)m);
-            const unsigned y1 = v + (unsigned)m < v ? v + (unsigned)m : v;  // v in [-m, m / 2]
-            const unsigned f = fh * (unsigned)y + __umulhi(fl, (unsigned)y);
-            if (!(scale_edges(y1 - yt, ylim, f) & lanes)) {
-                y = (int)y1;
-                st++;
-                continue;
-            }
-        }
-        // every later step maps 0 to 0
-        if ((long long)st * THRESH >= xbits && group_all(g, !act || y == 0)) break;
-        y = scale_step_reference(y, r, w, act ? c->pow2_inv[j - 1][g.gl] : 0, m, dinv, bad);
-        canon = group_all(g, !act || (unsigned)y < (unsigned)m);
-        st++;
-    }
-    replay_ok = !group_any(g, bad);
-    return y;
 }
 
 GRNS_D er_t bcast_er(er_t v, int lane) {

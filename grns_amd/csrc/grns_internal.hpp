@@ -94,3 +94,10 @@ inline size_t div_lanes_min(const grns_ctx *c) { return c->n > 16 ? 32768 : 1638
 // Lane-per-pair division (grns_divide.hip): pairs it does not take go to the rare queue.
 grns_status matrix_div(grns_ctx *c, const int *x, const int *d, long long smod, long long snum, size_t count, int *q,
                        int *r, const grns::RareQ &rq, hipStream_t s);
+// Scalings of at least this many numbers take their digits from the matrix cores (grns_scale.hip), 32
+// numbers to a wave; shorter ones a wave group per number.  By groups and by 32s, 16384 numbers of 8,
+// 16, 32, 64 moduli take 9, 16, 24, 54 us and 10, 18, 38, 83 us; 32768 take 12, 27, 39, 98 us and 10,
+// 18, 38, 87 us.
+constexpr size_t SCALE_MATRIX_MIN = 32768;
+grns_status matrix_scale(grns_ctx *c, const int *x, long long smod, long long snum, const unsigned *D, size_t count,
+                         int *y, hipStream_t s);

@@ -1874,109 +1874,264 @@ GRNS_D int group_rank_fast(const DevCtx *c, const Group &g, int s) {
     double fu = act ? dmul_ru((double)s, c->ru[g.gl]) : 0.0;
     return (int)group_psum<true>(g, fu);
 }
-// make_scaling_step, src/rnsscal.cuh:67-85 (j in [1, 30], pow2j = 2^j)
-GRNS_D int group_scaling_step(const DevCtx *c, const Group &g, int k, int j, int xi, int ci) {
+// make_scaling_step, src/rnsscal.cuh:67-85 (j in [1, 30], pow2j = 2^j), with the rank as rns_scale2pow takes
+// it.  The reference sums the terms of the residue modulo 2^j in 64 bits and reduces with `%`; modulo 2^j
+// the low 32 bits give the same integer.  `wraps`: some lane's result wraps int32.
+GRNS_D int group_scaling_step(const DevCtx *c, const Group &g, bool first, int j, int y, int &residue, bool &wraps) {
     const bool act = g.gl < g.L;
     const int mi = act ? c->m[g.gl] : 1;
     const double dinv = act ? c->dinv[g.gl] : 1.0;
-    const long long pow2j = 1ll << j;
-    long long term = 0;
-    if (act) {
-        long long prod = (long long)c->part_pow2_res[j - 1][g.gl] * (long long)ci;
-        // C's truncating remainder by a power of two
-        term = prod >= 0 ? (prod & (pow2j - 1)) : -((-prod) & (pow2j - 1));
-    }
-    long long residue = group_sum_ll(g, term);
-    long long temp = (long long)k * (long long)c->prod_pow2_res[j - 1];
-    residue = (residue - temp) % pow2j;
-    if (residue < 0) residue += pow2j;
-    int multiple = act ? (int)(residue % mi) : 0;
-    multiple = act ? psubmod(xi, multiple, mi, dinv) : 0;
-    return act ? mulmod_recip(multiple, c->pow2_inv[j - 1][g.gl], mi, dinv) : 0;
-}
-// rns_scale2pow, src/rnsscal.cuh:93-119
-GRNS_D int group_scale2pow(const DevCtx *c, const Group &g, int xi, unsigned D) {
-    const bool act = g.gl < g.L;
-    const int mi = act ? c->m[g.gl] : 1;
-    const double dinv = act ? c->dinv[g.gl] : 1.0;
-    const int w = act ? c->w[g.gl] : 0;
-    int result = xi;
-    int t = (int)(D / THRESH);
-    int k;
-    if (t > 0) {
-        int ci = act ? mulmod_recip(xi, w, mi, dinv) : 0;
-        k = group_rank(c, g, xi, ci);
-        result = group_scaling_step(c, g, k, THRESH, xi, ci);
-        t -= 1;
-    }
-    while (t > 0) {
-        // a step maps residues that are all 0 to all 0 (c = 0, rank 0, remainder 0): once there, the
-        // remaining steps of the reference change nothing, which bounds the loop for any D
-        if (group_all(g, !act || result == 0)) break;
-        int ci = act ? mulmod_recip(result, w, mi, dinv) : 0;
-        k = group_rank_fast(c, g, ci);
-        result = group_scaling_step(c, g, k, THRESH, result, ci);
-        t -= 1;
-    }
-    unsigned d = D % THRESH;
-    if (d > 0) {
-        int ci = act ? mulmod_recip(result, w, mi, dinv) : 0;
-        k = d < D ? group_rank_fast(c, g, ci) : group_rank(c, g, result, ci);
-        result = group_scaling_step(c, g, k, (int)d, result, ci);
-    }
-    return result;
+    const int ci = act ? mulmod_recip(y, c->w[g.gl], mi, dinv) : 0;
+    const int k = first ? group_rank(c, g, y, ci) : group_rank_fast(c, g, ci);
+    unsigned sum = act ? (unsigned)c->part_pow2_res[j - 1][g.gl] * (unsigned)ci : 0u;
+    for (int s = 1; s < g.G; s <<= 1) sum += (unsigned)__shfl_xor((int)sum, s, 64);
+    residue = (int)((sum - (unsigned)k * (unsigned)c->prod_pow2_res[j - 1]) & ((1u << j) - 1u));
+    const int mult = psubmod(y, (int)rem_trunc_d((long long)residue, (double)residue, mi, dinv), mi, dinv);
+    const int inv = act ? c->pow2_inv[j - 1][g.gl] : 0;
+    const int qi = (int)(((double)mult * (double)inv) * dinv);
+    const long long v = (long long)mult * inv - (long long)qi * mi;
+    wraps = group_any(g, v < -2147483648ll || v > 2147483647ll);
+    return (int)v;
 }
 
-// Scaling of canonical numbers by the replayed word form; the others (non-canonical residues, a
-// replay that meets an int32 wrap) go to the rare queue for the reference steps.
+// One step of the replay below as the reference computes it, for any y it may hold: X_s mod 2^j is
+// r, inv is (2^j)^-1 mod m.  `bad`: c = y w is not canonical, or y' wraps int32.
+GRNS_D int scale_step_reference(int y, unsigned r, int w, int inv, int m, double dinv, bool &bad) {
+    const int cc = mulmod_recip(y, w, m, dinv);
+    bad |= (unsigned)cc >= (unsigned)m;
+    // rm = r % m and mult = (y - rm + m) % m as rem_trunc forms them: r < 2^30 and
+    // |y - rm + m| < 2^32 have exact doubles, formed from 32-bit pieces
+    const int rm = (int)rem_trunc_d((long long)r, (double)r, m, dinv);
+    const int mult = (int)rem_trunc_d((long long)y + (m - rm), (double)y + (double)(m - rm), m, dinv);
+    const int qi = (int)(((double)mult * (double)inv) * dinv);
+    const long long v = (long long)mult * inv - (long long)qi * m;
+    bad |= v < -2147483648ll || v > 2147483647ll;
+    return (int)v;
+}
+
+// Bits [30 l, 30 l + 30) of the group's value, l >= 0 the lane's own choice.
+template <int GD>
+GRNS_D unsigned digit30(const Group &g, unsigned X, int l) {
+    const int b = 30 * l, w0 = b >> 5, sh = b & 31;
+    unsigned lo = (unsigned)__shfl((int)X, g.base + (w0 < GD ? w0 : 0), 64);
+    unsigned hi = (unsigned)__shfl((int)X, g.base + (w0 + 1 < GD ? w0 + 1 : 0), 64);
+    lo = w0 < GD ? lo : 0u;
+    hi = w0 + 1 < GD ? hi : 0u;
+    return (unsigned)((((unsigned long long)hi << 32) | lo) >> sh) & 0x3fffffffu;
+}
+
+// The active lanes whose y' (yo = y' - rec_t) or fraction of y w / m (f + 4100 in 32 bits, at most 2
+// below the true one) is too near the edges: both limits keep a fraction 2^-20 from an integer.  yo
+// and f may be the largest of several steps.
+GRNS_D unsigned long long scale_edges(unsigned yo, unsigned ylim, unsigned f) {
+    return __builtin_amdgcn_uicmp(yo, ylim, 35) | __builtin_amdgcn_uicmp(f, 0u - 8200u, 35);  // ICMP_UGE
+}
+
+// A value that is the same in all lanes of a group, held in scalar registers when the group is the wave.
+template <int GD>
+GRNS_D int group_uniform(int v) {
+    return GD == 64 ? __builtin_amdgcn_readfirstlane(v) : v;
+}
+
+// The lane's constants of the replay.  Lanes past n take no part (m = 1, w = 0, inverses 0).
+struct ScaleLane {
+    int m, w;
+    unsigned minv, fh, fl, yt, ylim;
+    double dinv;
+    unsigned long long lanes;  // the group's active lanes
+    bool odd;                  // every modulus is odd
+    bool large;                // and at least 2^20
+};
+GRNS_D ScaleLane scale_lane(const DevCtx *c, const Group &g) {
+    const bool act = g.gl < g.L;
+    ScaleLane k;
+    k.m = act ? c->m[g.gl] : 1;
+    k.w = act ? c->w[g.gl] : 0;
+    k.dinv = act ? c->dinv[g.gl] : 1.0;
+    k.minv = act ? c->minv[g.gl] : 0u;
+    k.fh = act ? c->wf_hi[g.gl] : 0u;
+    k.fl = act ? c->wf_lo[g.gl] : 0u;
+    k.yt = act ? c->rec_t[g.gl] : 0u;
+    k.ylim = act ? c->rec_lim[g.gl] : 0u;
+    k.lanes = __ballot(act) & group_mask_bits(g);
+    k.odd = c->odd_moduli != 0;
+    k.large = k.odd && c->m_min >= (1 << 20);
+    return k;
+}
+
+// rns_scale2pow (src/rnsscal.cuh:93-119) replayed on the digits of a canonical x.  Step s of the
+// reference maps its value X_s = floor(x / 2^(30 s)) to X_{s+1} = floor(X_s / 2^j): with its
+// residues y (as the reference holds them, possibly y + m or y - m) it forms c = y * w (for the
+// rank), X_s mod 2^j, multiple = (y - (X_s mod 2^j) mod m + m) % m and y' = multiple * (2^j)^-1,
+// the products by reciprocal reduction.  Whenever every c is canonical, the rank and the residue
+// X_s mod 2^j of the reference are consistent, so X_s mod 2^j is the bits [30 s, 30 s + j) of x, and
+// y' follows from y exactly as the reference computes it.  A step whose c is not canonical forms rank and
+// residue as the reference does; where they give other bits, and where y' wraps int32 (the reference
+// then continues with another number), the replay ends: y is what the reference holds after the
+// first `st` steps, and the caller goes on with the reference's steps.
+//
+// A reciprocal product is canonical unless its fraction is within 2^-20.4 of an integer.  So steps
+// from canonical y first take y' by exact division, y' = (y - r) / 2^j mod m = (d - h m) / 2^j
+// with d = y - r and h = d m^-1 mod 2^j (two 32-bit multiplications: the low parts of d and h m are
+// equal, so the high parts alone give the quotient), and the fraction of y w / m to 32 bits (two
+// more): when every lane's y' and fraction keep their distance from the edges, the reference's
+// products are canonical and y' is its result.  Four full steps, where the moduli are large, or all
+// that are left, share one check; where it fails (one step in about 10^4, and those near the end of a
+// small value) the steps are taken one by one, and one that fails alone runs as the reference computes it.
+// So does every step of a set with an even modulus, which has no inverse of 2.
+//
+// xg: the group's x; dig(s): bits [30 s, 30 s + 30) of x (0 past its end); dig4(s, r): four of them from
+// s <= 2 GD on, s a multiple of 4; xbits: x is below 2^xbits.
+template <int GD, class Dig, class Dig4>
+GRNS_D void scale_replay(const DevCtx *c, const Group &g, const ScaleLane &k, unsigned D, int xbits, Dig dig, Dig4 dig4,
+                         int &y, unsigned &st) {
+    const bool act = g.gl < g.L, fast = k.odd;
+    const unsigned t = D / THRESH, dr = D % THRESH;
+    const unsigned steps = t + (dr ? 1u : 0u);
+    const unsigned some = t < 2 * GD ? t & ~3u : 2 * GD;  // from digit 2 GD on x is 0
+    const unsigned fours = k.large ? some : 0u;
+    bool canon = group_all(g, !act || (unsigned)y < (unsigned)k.m), rest = fast;
+    const unsigned um = (unsigned)k.m, nminv30 = 0u - (k.minv << (32 - THRESH));
+    auto fraction = [&](unsigned v) { return k.fh * v + __umulhi(k.fl, v) - 4100u; };
+    auto exact = [&](unsigned v, unsigned r, int j) {
+        const int d = (int)(v - r);
+        const unsigned q = (unsigned)(d >> j) - __umulhi(((unsigned)d * k.minv) << (32 - j), um);  // in [-m, m / 2]
+        return q + um < q ? q + um : q;
+    };
+    auto digit = [&](unsigned s, int j) { return dig((int)s) & ((1u << j) - 1u); };
+    while (st < steps) {
+        if (canon && !(st & 3u) && st < fours) {
+            unsigned r[4];
+            dig4((int)st, r);
+            for (; st < fours; st += 4) {
+                unsigned next[4], yo = 0, fo = 0, v = (unsigned)y;
+                dig4((int)st + 4, next);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const unsigned f = fraction(v);
+                    const int d = (int)(v - r[i]);
+                    // h = 0 gives 1 or 2 here: below rec_t
+                    v = __umulhi((unsigned)d * nminv30, um) + (unsigned)(d >> THRESH) + 1u;
+                    const unsigned o = v - k.yt;
+                    yo = o > yo ? o : yo;
+                    fo = f > fo ? f : fo;
+                }
+                if (scale_edges(yo, k.ylim, fo) & k.lanes) break;
+                y = (int)v;
+#pragma unroll
+                for (int i = 0; i < 4; i++) r[i] = next[i];
+            }
+            if (st >= steps) break;
+        }
+        if (canon && rest && st + 4 >= steps) {
+            rest = false;
+            unsigned yo = 0, fo = 0, v = (unsigned)y;
+            for (unsigned s = st; s < steps; s++) {
+                const int j = (s < t) ? THRESH : (int)dr;
+                const unsigned f = fraction(v);
+                v = exact(v, digit(s, j), j);
+                const unsigned o = v - k.yt;
+                yo = o > yo ? o : yo;
+                fo = f > fo ? f : fo;
+            }
+            if (!(scale_edges(yo, k.ylim, fo) & k.lanes)) {
+                y = (int)v;
+                st = steps;
+                break;
+            }
+        }
+        const int j = (st < t) ? THRESH : (int)dr;
+        const unsigned r = digit(st, j);
+        if (fast && canon) {
+            const unsigned y1 = exact((unsigned)y, r, j);
+            if (!(scale_edges(y1 - k.yt, k.ylim, fraction((unsigned)y)) & k.lanes)) {
+                y = (int)y1;
+                st++;
+                continue;
+            }
+        }
+        // every later step maps 0 to 0
+        if ((long long)st * THRESH >= xbits && group_all(g, !act || y == 0)) {
+            st = steps;
+            break;
+        }
+        bool bad = false;
+        const int y1 = scale_step_reference(y, r, k.w, act ? c->pow2_inv[j - 1][g.gl] : 0, k.m, k.dinv, bad);
+        if (group_any(g, bad)) break;
+        y = y1;
+        canon = group_all(g, !act || (unsigned)y1 < um);
+        st++;
+    }
+}
+
+// rns_scale2pow of x: the replay (`follow`: x is canonical), and steps as the reference takes them
+// where it stops.  After such a step whose residue is x's digit, the replay goes on.  A step of
+// residues that are all 0 gives all 0 (c = 0, rank 0, remainder 0): the remaining ones change nothing, which
+// bounds the loop for any D.
+template <int GD, class Dig, class Dig4>
+GRNS_D int group_scale_digits(const DevCtx *c, const Group &g, const ScaleLane &k, int xi, unsigned D, int xbits,
+                              bool follow, Dig dig, Dig4 dig4) {
+    const unsigned t = D / THRESH, dr = D % THRESH;
+    int y = g.gl < g.L ? xi : 0;
+    for (unsigned st = 0; st < t + (dr ? 1u : 0u); st++) {
+        if (follow) {
+            scale_replay<GD>(c, g, k, D, xbits, dig, dig4, y, st);
+            if (st >= t + (dr ? 1u : 0u)) break;
+        }
+        bool wraps;
+        int residue;
+        const int j = st < t ? THRESH : (int)dr;
+        if (st && group_all(g, y == 0)) break;
+        y = group_scaling_step(c, g, st == 0, j, y, residue, wraps);
+        follow = group_uniform<GD>(follow && !wraps && residue == (int)(dig((int)st) & ((1u << j) - 1u)));
+    }
+    return y;
+}
+
+// rns_scale2pow on the words of x (group of GD lanes): the lanes hold the 30-bit digits.
+template <int GD>
+GRNS_D int group_scale2pow_words(const DevCtx *c, const Group &g, int xi, unsigned D) {
+    D = (unsigned)group_uniform<GD>((int)D);
+    const bool canonical = group_all(g, g.gl >= g.L || (unsigned)xi < (unsigned)c->m[g.gl]);
+    const unsigned X = canonical ? group_words<GD>(c, g, xi) : 0u;
+    const unsigned dig0 = digit30<GD>(g, X, g.gl), dig1 = digit30<GD>(g, X, g.gl + GD);
+    auto dig = [&](int s) {
+        return s < GD ? gword<GD>(g, dig0, s) : s < 2 * GD ? gword<GD>(g, dig1, s - GD) : 0u;
+    };
+    return group_scale_digits<GD>(c, g, scale_lane(c, g), xi, D, 32 * wlen<GD>(g, X), canonical, dig, [&](int s, unsigned(&r)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = s + 4 <= GD ? gword<GD>(g, dig0, s + i) : dig(s + i);
+    });
+}
+// The reference's steps alone.
+GRNS_D int group_scale2pow(const DevCtx *c, const Group &g, int y, unsigned D) {
+    const unsigned t = D / THRESH, dr = D % THRESH;
+    for (unsigned st = 0; st < t + (dr ? 1u : 0u); st++) {
+        bool wraps;
+        int residue;
+        if (st && group_all(g, g.gl >= g.L || y == 0)) break;
+        y = group_scaling_step(c, g, st == 0, st < t ? THRESH : (int)dr, y, residue, wraps);
+    }
+    return y;
+}
+
+// Scaling by the replayed word form, a wave group per number.
 template <int GD>
 __global__ __launch_bounds__(BLOCK) void k_scale2pow_words(const DevCtx *__restrict__ c, const int *__restrict__ x,
                                                            long long smod, long long snum,
                                                            const unsigned *__restrict__ D, long long count,
-                                                           int *__restrict__ y, RareQ rq) {
+                                                           int *__restrict__ y) {
     const Group g = make_group(GD, c->n);
     constexpr int P = 64 / GD;
     const long long wave = ((long long)xcd_block() * BLOCK + threadIdx.x) >> 6;
     const long long nwaves = ((long long)gridDim.x * BLOCK) >> 6;
     for (long long j0 = wave * P; j0 < count; j0 += nwaves * P) {
         const long long j = j0 + (threadIdx.x & 63) / GD;
-        const bool valid = j < count;
-        bool ok = false;
-        if (valid) {
-            const bool act = g.gl < g.L;
+        if (j < count) {
             const long long off = j * snum + (long long)g.gl * smod;
-            const int xi = act ? x[off] : 0;
-            if (group_all(g, !act || (unsigned)xi < (unsigned)c->m[g.gl])) {
-                const int v = group_scale2pow_words<GD>(c, g, xi, D[j], ok);
-                if (ok && act) y[off] = v;
-            }
+            const int v = group_scale2pow_words<GD>(c, g, g.gl < g.L ? x[off] : 0, D[j]);
+            if (g.gl < g.L) y[off] = v;
         }
-        const bool rare = valid && !ok && g.gl == 0;
-        if (!rare_push(rq, rare, j)) y[j * snum] = DIV_MARK;
-    }
-}
-
-// Rare pass of the scaling: the reference steps, one wave group per queued number (and, after a
-// queue overflow, per marked number).
-static __global__ __launch_bounds__(BLOCK) void k_scale2pow_rare(const DevCtx *__restrict__ c, int G, const int *__restrict__ x,
-                                                          long long smod, long long snum, const unsigned *__restrict__ D,
-                                                          long long count, int *__restrict__ y, RareQ rq) {
-    Group g = make_group(G, c->n);
-    const int P = 64 / G;
-    const long long gid = (((long long)blockIdx.x * BLOCK + threadIdx.x) >> 6) * P + (threadIdx.x & 63) / G;
-    const long long ngroups = ((long long)gridDim.x * BLOCK >> 6) * P;
-    __shared__ RareView v;
-    rare_view(rq, v);
-    const long long nq = v.pre[RARE_SUBQ];
-    const long long total = nq + (rq.ctr[2] ? count : 0);
-    for (long long k = gid; k < total; k += ngroups) {
-        const int *unused;
-        const long long j = rare_item(rq, v, k, unused);
-        if (k >= nq && y[j * snum] != DIV_MARK) continue;
-        const long long off = j * snum + (long long)g.gl * smod;
-        const int xi = g.gl < g.L ? x[off] : 0;
-        const int v = group_scale2pow(c, g, xi, D[j]);
-        if (g.gl < g.L) y[off] = v;
     }
 }
 
