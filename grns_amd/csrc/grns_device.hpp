@@ -575,6 +575,13 @@ GRNS_HD double psum_one(Leaf &leaf) {
     }
 }
 
+// Orders the wave's own LDS accesses: what any lane wrote before is read by every lane after.
+GRNS_D void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------- wave groups (N lanes per number)
 // A group is G = 2^g >= N consecutive lanes of a wave64, aligned on G; lane gl of a group holds
 // modulus gl.  Cross-lane traffic stays inside the group.

@@ -560,6 +560,11 @@ grns_status grns_eval(grns_ctx *c, const int *x, long long smod, long long snum,
                                          cnt, o, q);                                                             \
             else hipLaunchKernelGGL((k_eval<NN, false, LD_MM>), grid, blk, 0, S(stream), c->d, x, smod, snum, cnt, \
                                     o, q);                                                                       \
+        } else if (smod == 1) {                                                                                  \
+            if (fast) hipLaunchKernelGGL((k_eval<NN, true, LD_NM>), grid, blk, 0, S(stream), c->d, x, smod, snum,  \
+                                         cnt, o, q);                                                             \
+            else hipLaunchKernelGGL((k_eval<NN, false, LD_NM>), grid, blk, 0, S(stream), c->d, x, smod, snum, cnt, \
+                                    o, q);                                                                       \
         } else {                                                                                                 \
             if (fast) hipLaunchKernelGGL((k_eval<NN, true, LD_ANY>), grid, blk, 0, S(stream), c->d, x, smod, snum, \
                                          cnt, o, q);                                                             \
@@ -619,6 +624,8 @@ grns_status grns_cmp(grns_ctx *c, const int *x, long long xsm, long long xsn, co
         int tk = stage_begin(c, 1, stream);                                                                        \
         if (mm) hipLaunchKernelGGL((k_cmp<NN, LD_MM>), grid, blk, 0, S(stream), c->d, x, xsm, xsn, y, ysm, ysn, cnt,  \
                                    sign, q);                                                                       \
+        else if (xsm == 1 && ysm == 1) hipLaunchKernelGGL((k_cmp<NN, LD_NM>), grid, blk, 0, S(stream), c->d, x, xsm,  \
+                                                          xsn, y, ysm, ysn, cnt, sign, q);                         \
         else hipLaunchKernelGGL((k_cmp<NN, LD_ANY>), grid, blk, 0, S(stream), c->d, x, xsm, xsn, y, ysm, ysn, cnt,     \
                                 sign, q);                                                                          \
         stage_end(c, 1, tk, stream);                                                                               \
@@ -713,9 +720,13 @@ grns_status grns_mrc(grns_ctx *c, const int *x, long long smod, long long snum, 
     }
     const long long cnt = (long long)count;
     dim3 blk(BLOCK), lgrid((unsigned)grid_elems(count));
+    const bool nm = (smod == 1 && snum != 1) || (dsm == 1 && dsn != 1);  // numbers side by side
 #define GRNS_MRC_CASE(NN)                                                                                         \
     case NN:                                                                                                      \
-        hipLaunchKernelGGL((k_mrc_lane<NN>), lgrid, blk, 0, S(stream), c->d, x, smod, snum, cnt, d, dsm, dsn);     \
+        if (nm) hipLaunchKernelGGL((k_mrc_lane<NN, true>), lgrid, blk, 0, S(stream), c->d, x, smod, snum, cnt, d, dsm, \
+                                   dsn);                                                                          \
+        else hipLaunchKernelGGL((k_mrc_lane<NN, false>), lgrid, blk, 0, S(stream), c->d, x, smod, snum, cnt, d, dsm,   \
+                                dsn);                                                                             \
         return launch_check();
     switch (c->n) {
         GRNS_MRC_CASE(4)
@@ -871,6 +882,8 @@ static grns_status max_run(grns_ctx *c, const int *x, long long smod, long long 
         if (timed) tk = stage_begin(c, 2, stream);                                                           \
         if (mm) hipLaunchKernelGGL((k_max_partial<NN, LD_MM>), grid, blk, 0, S(stream), c->d, x, smod, snum, \
                                    cnt, ch, part, part_res);                                                 \
+        else if (smod == 1) hipLaunchKernelGGL((k_max_partial<NN, LD_NM>), grid, blk, 0, S(stream), c->d, x,   \
+                                               smod, snum, cnt, ch, part, part_res);                         \
         else hipLaunchKernelGGL((k_max_partial<NN, LD_ANY>), grid, blk, 0, S(stream), c->d, x, smod, snum,    \
                                 cnt, ch, part, part_res);                                                    \
         if (timed) stage_end(c, 2, tk, stream);                                                              \
@@ -937,10 +950,13 @@ grns_status grns_max_mrc(grns_ctx *c, const int *x, long long smod, long long sn
     int *pdig = reinterpret_cast<int *>(pidx + nb);
     dim3 grid((unsigned)nb), blk(BLOCK);
     long long cnt = (long long)count;
+    const bool nm = smod == 1 && snum != 1;
 #define GRNS_MAX_MRC_CASE(NN)                                                                                   \
     case NN:                                                                                                    \
-        hipLaunchKernelGGL((k_max_mrc_partial<NN>), grid, blk, 0, S(stream), c->d, x, smod, snum, cnt, ch, pidx,   \
-                           pdig);                                                                               \
+        if (nm) hipLaunchKernelGGL((k_max_mrc_partial<NN, true>), grid, blk, 0, S(stream), c->d, x, smod, snum, cnt,  \
+                                   ch, pidx, pdig);                                                             \
+        else hipLaunchKernelGGL((k_max_mrc_partial<NN, false>), grid, blk, 0, S(stream), c->d, x, smod, snum, cnt,    \
+                                ch, pidx, pdig);                                                                \
         if (hipGetLastError() != hipSuccess) return GRNS_ERR_HIP;                                               \
         hipLaunchKernelGGL((k_max_mrc_final<NN>), dim3(1), blk, 0, S(stream), x, smod, snum, pidx, pdig, (int)nb, \
                            out_residues, out_idx);                                                              \

@@ -78,13 +78,6 @@ GRNS_D v16i load_init(const int *p) {
     return a;
 }
 
-// Orders the wave's own LDS accesses: what any lane wrote before is read by every lane after.
-GRNS_D void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Value of another lane's register 32 lanes away.
 GRNS_D int other_half(int v) { return __shfl_xor(v, 32, 64); }
 GRNS_D double other_half_d(double v) { return __shfl_xor(v, 32, 64); }
