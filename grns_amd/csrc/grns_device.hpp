@@ -1157,13 +1157,14 @@ GRNS_D void group_refine(const DevCtx *c, const Group &g, int &s, double sumu, i
     int kprev = -1, p2 = 0;
     while (sumu < c->accuracy) {
         // MAX(-(ceil(log2(sumu))+1), REF): log2 of a negative sum is NaN and selects REF; a zero
-        // sum gives +inf, which the reference turns into an index outside RNS_POW2.
+        // sum gives +inf, and REF of a single modulus (whose accuracy is 0) is -inf: the reference turns
+        // both into an index outside RNS_POW2.
         double kv = (double)c->ref_factor;
         if (sumu > 0) {
             double a = (double)(-(ceil_log2_libm(sumu) + 1));
             kv = a > kv ? a : kv;
         }
-        if (sumu == 0 || kv > c->log2M || ++it > 4096) {
+        if (sumu == 0 || kv < 0 || kv > c->log2M || ++it > 4096) {
             status |= GST_REFINE;
             out.low.frac = out.upp.frac = __builtin_nan("");
             out.low.exp = out.upp.exp = 0;

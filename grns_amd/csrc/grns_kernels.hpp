@@ -832,7 +832,7 @@ GRNS_HD void refine_lane(const DevCtx *c, int (&s)[N], double sumu, interval_t &
             double a = (double)(-(ceil_log2_libm(sumu) + 1));
             kv = a > kv ? a : kv;
         }
-        if (sumu == 0 || kv > c->log2M || ++it > 4096) {
+        if (sumu == 0 || kv < 0 || kv > c->log2M || ++it > 4096) {
             status |= GST_REFINE;
             out.low.frac = out.upp.frac = __builtin_nan("");
             out.low.exp = out.upp.exp = 0;

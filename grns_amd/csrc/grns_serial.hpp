@@ -93,7 +93,7 @@ GRNS_D void serial_refine(const DevCtx *c, int *s, double sumu, interval_t &out,
             double a = (double)(-(ceil_log2_libm(sumu) + 1));
             kv = a > kv ? a : kv;
         }
-        if (sumu == 0 || kv > c->log2M || ++it > 4096) {  // the reference reads outside RNS_POW2
+        if (sumu == 0 || kv < 0 || kv > c->log2M || ++it > 4096) {  // the reference reads outside RNS_POW2
             status |= GST_REFINE;
             out.low.frac = out.upp.frac = __builtin_nan("");
             out.low.exp = out.upp.exp = 0;
