@@ -160,8 +160,7 @@ GRNS_D void for_group_tiles(const DevCtx *c, int G, const BatchTask *__restrict_
     }
 }
 
-// Division (group of GD lanes per pair): the word division, or the reference loop for the pairs it
-// does not take.
+// Division (group of GD lanes per pair).
 template <int GD>
 __global__ __launch_bounds__(BLOCK) void k_batch_div(const DevCtx *__restrict__ c, const BatchTask *__restrict__ tasks,
                                                      int ntasks, long long total, int tile,
@@ -169,12 +168,8 @@ __global__ __launch_bounds__(BLOCK) void k_batch_div(const DevCtx *__restrict__ 
     for_group_tiles(c, GD, tasks, ntasks, total, tile, counter, [&](const BatchTask &T, const Group &g, long long j) {
         const bool act = g.gl < g.L;
         const long long oa = j * T.asn + (long long)g.gl * T.asm_;
-        const int xi = act ? T.a[oa] : 0;
-        const int di = act ? T.b[oa] : 0;
         int q, r, st = 0;
-        if (div_words_ok(c, g, xi, di)) group_div_words<GD>(c, g, xi, di, q, r);
-        else if (T.op == GRNS_OP_DIV) group_div<false>(c, g, xi, di, q, r, st);
-        else group_div<true>(c, g, xi, di, q, r, st);
+        group_div_any<GD>(c, g, act ? T.a[oa] : 0, act ? T.b[oa] : 0, T.op == GRNS_OP_DIV_FAST, q, r, st);
         if (act) {
             reinterpret_cast<int *>(T.o0)[oa] = q;
             reinterpret_cast<int *>(T.o1)[oa] = r;

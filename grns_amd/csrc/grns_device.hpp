@@ -191,6 +191,16 @@ GRNS_HD double dmul_rd(double a, double b) { double c = a * b; return c - bn_err
 GRNS_HD double dmul_ru(double a, double b) { double c = a * b; return c + bn_err(c); }
 GRNS_HD double ddiv_rd(double a, double b) { double c = a / b; return c - bn_err(c); }
 GRNS_HD double ddiv_ru(double a, double b) { double c = a / b; return c + bn_err(c); }
+// RN(s / m) of integers below 2^32 from y = RN(1 / m): s y is within 2 ulp of the quotient, the first
+// correction brings it within 1 ulp, and from there (Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990, theorem 8.1) the second one is correctly
+// rounded.  Five operations instead of the thirteen of a division.
+GRNS_HD double quot_rn(double s, double m, double y) {
+    const double q = s * y, q1 = fma(fma(-q, m, s), y, q);
+    return fma(fma(-q1, m, s), y, q1);
+}
+GRNS_HD double quot_rd(double s, double m, double y) { double c = quot_rn(s, m, y); return c - bn_err(c); }
+GRNS_HD double quot_ru(double s, double m, double y) { double c = quot_rn(s, m, y); return c + bn_err(c); }
 
 template <bool UP> GRNS_HD double dadd_dir(double a, double b) { return UP ? dadd_ru(a, b) : dadd_rd(a, b); }
 
@@ -607,8 +617,63 @@ GRNS_D int bcast_i(int v, int lane) { return __shfl(v, lane, 64); }
 GRNS_D double bcast_d(double v, int lane) { return __shfl(v, lane, 64); }
 GRNS_D long long bcast_ll(long long v, int lane) { return __shfl(v, lane, 64); }
 
-// Pairwise tree over the group's leaves in the CPU association (xor butterfly; an absent second
-// half contributes the literal 0 of src/pairwise.cuh, an absent first half makes the node absent).
+// The values of the lower and the upper half of the lane's block of 2 H lanes (H = 1, 2, .., 32), for a
+// value that is the same on all lanes of a half: within rows of 16 by DPP (a mirrored row serves for
+// H = 4 and 8), across rows by a swap of rows.  A shuffle through LDS takes about
+// ten times as long, and trees over a group wait for one per level.
+template <int H>
+GRNS_D void lane_halves(unsigned v, int gl, unsigned &lo, unsigned &hi) {
+    if constexpr (H >= 16) {
+        const auto r = H == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                               : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        lo = r[0];
+        hi = r[1];
+    } else {
+        // quad_perm 1,0,3,2; quad_perm 2,3,0,1; row_half_mirror; row_mirror
+        constexpr int CTRL = H == 1 ? 0xB1 : H == 2 ? 0x4E : H == 4 ? 0x141 : 0x140;
+        const unsigned w = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+        const bool upper = (gl & H) != 0;
+        lo = upper ? w : v;
+        hi = upper ? v : w;
+    }
+}
+template <int H>
+GRNS_D void lane_halves(unsigned long long v, int gl, unsigned long long &lo, unsigned long long &hi) {
+    unsigned l0, h0, l1, h1;
+    lane_halves<H>((unsigned)v, gl, l0, h0);
+    lane_halves<H>((unsigned)(v >> 32), gl, l1, h1);
+    lo = (unsigned long long)l1 << 32 | l0;
+    hi = (unsigned long long)h1 << 32 | h0;
+}
+template <int H>
+GRNS_D void lane_halves(double v, int gl, double &lo, double &hi) {
+    unsigned long long l, u;
+    lane_halves<H>((unsigned long long)__double_as_longlong(v), gl, l, u);
+    lo = __longlong_as_double((long long)l);
+    hi = __longlong_as_double((long long)u);
+}
+
+// Pairwise tree over the group's leaves in the CPU association (an absent second half contributes the
+// literal 0 of src/pairwise.cuh, an absent first half makes the node absent): the levels from H on, up to
+// K lanes.
+template <bool UP, int H>
+GRNS_D double psum_levels(const Group &g, int K, double v) {
+    if constexpr (H <= 64) {
+        if (H < K) {
+            const int b = g.gl & ~(2 * H - 1);
+            double fv = v, sv = 0.0;
+            if constexpr (H < 64) {
+                if (H < g.G) {
+                    lane_halves<H>(v, g.gl, fv, sv);
+                    sv = b + H < g.L ? sv : 0.0;
+                }
+            }
+            const double r = dadd_dir<UP>(fv, sv);
+            v = psum_levels<UP, 2 * H>(g, K, b < g.L ? r : v);
+        }
+    }
+    return v;
+}
 template <bool UP>
 GRNS_D double group_psum(const Group &g, double v) {
     const int L = g.L;
@@ -619,16 +684,17 @@ GRNS_D double group_psum(const Group &g, double v) {
     }
     int K = 2;
     if (L >= 4) { K = 8; while (K <= L) K <<= 1; }
-    for (int h = 1; h < K; h <<= 1) {
-        double w = (h < g.G) ? __shfl_xor(v, h, 64) : 0.0;
-        int b = g.gl & ~(2 * h - 1);
-        bool first = b < L;
-        bool second = (h < g.G) && (b + h < L);
-        bool upper = (g.gl & h) != 0;
-        double fv = upper ? w : v;
-        double sv = second ? (upper ? v : w) : 0.0;
-        double r = dadd_dir<UP>(fv, sv);
-        v = first ? r : v;
+    return psum_levels<UP, 1>(g, K, v);
+}
+// Sums over the group.
+template <int H = 1, class T>
+GRNS_D T group_sum(const Group &g, T v) {
+    if constexpr (H < 64) {
+        if (H < g.G) {
+            T lo, hi;
+            lane_halves<H>(v, g.gl, lo, hi);
+            v = group_sum<2 * H>(g, lo + hi);
+        }
     }
     return v;
 }
@@ -659,14 +725,6 @@ GRNS_HD int class_order(int kx, long long Tx, int ky, long long Ty) {
 
 // Wave-group forms of the certificates: lane gl holds residue gl; the sums run over the group in
 // any order (the certificates verify what they find, and the filter bound holds for any order).
-GRNS_D double group_sum_d(const Group &g, double v) {
-    for (int h = 1; h < g.G; h <<= 1) v += __shfl_xor(v, h, 64);
-    return v;
-}
-GRNS_D unsigned long long group_sum_u64(const Group &g, unsigned long long v) {
-    for (int h = 1; h < g.G; h <<= 1) v += (unsigned long long)__shfl_xor((long long)v, h, 64);
-    return v;
-}
 
 // crt_rep for the group's number with canonical residue di: the representative T of x within 2^62
 // of 0 or M (x = T or M + T), verified against every residue.
@@ -685,8 +743,8 @@ GRNS_D bool group_crt_rep(const DevCtx *c, const Group &g, int di, long long &Ts
         a = s * c->dinv[i];
         t = (unsigned long long)(unsigned)(int)s * c->mi64[i];
     }
-    const double acc = group_sum_d(g, a);
-    const unsigned long long T = group_sum_u64(g, t) - (unsigned long long)(long long)rint(acc) * c->M64;
+    const double acc = group_sum(g, a);
+    const unsigned long long T = group_sum(g, t) - (unsigned long long)(long long)rint(acc) * c->M64;
     Ts = (long long)T;
     if (Ts >= (1ll << 62) || Ts <= -(1ll << 62)) return false;
     bool ok = true;
@@ -716,7 +774,7 @@ GRNS_D double group_filter(const DevCtx *c, const Group &g, int xi, bool &canon,
         fi = fract_d(P) + t;
         tm = fabs(fi - 0.5) < 0.5 - 0x1p-20;
     }
-    const double F = fract_d(group_sum_d(g, fi));
+    const double F = fract_d(group_sum(g, fi));
     canon = group_all(g, cn);
     terms = group_all(g, tm);
     return F;
@@ -1013,7 +1071,7 @@ GRNS_D unsigned group_words(const DevCtx *c, const Group &g, int xi) {
     const bool act = g.gl < g.L;
     const double dinv = act ? c->dinv[g.gl] : 1.0;
     const int s[1] = {act ? mulmod3(xi, c->w[g.gl], c->m[g.gl], dinv) : 0};
-    const double sum = group_sum_d(g, act ? (double)s[0] * dinv : 0.0);
+    const double sum = group_sum(g, act ? (double)s[0] * dinv : 0.0);
     unsigned long long lo[1], hi[1];
     crt_columns<GD, 1>(c, g, s, lo, hi);
     return crt_finish<GD>(c, g, lo[0], hi[0], sum);
@@ -1031,8 +1089,8 @@ GRNS_D void group_words_pair(const DevCtx *c, const Group &g, int xi, int di, un
         dinv = c->dinv[g.gl];
     }
     const int s[2] = {act ? mulmod3(xi, w, m, dinv) : 0, act ? mulmod3(di, w, m, dinv) : 0};
-    const double sx = group_sum_d(g, act ? (double)s[0] * dinv : 0.0);
-    const double sd = group_sum_d(g, act ? (double)s[1] * dinv : 0.0);
+    const double sx = group_sum(g, act ? (double)s[0] * dinv : 0.0);
+    const double sd = group_sum(g, act ? (double)s[1] * dinv : 0.0);
     unsigned long long lo[2], hi[2];
     crt_columns<GD, 2>(c, g, s, lo, hi);
     X = crt_finish<GD>(c, g, lo[0], hi[0], sx);
@@ -1176,12 +1234,12 @@ GRNS_D void group_refine(const DevCtx *c, const Group &g, int &s, double sumu, i
             kprev = k;
         }
         s = mulmod_recip(s, p2, mi, dinv);
-        double fu = ddiv_ru((double)s, dm);
+        double fu = quot_ru((double)s, dm, dinv);
         sumu = group_psum<true>(g, fu);
         sumu -= to_uint(sumu);
         K += k;
     }
-    double fl = ddiv_rd((double)s, dm);
+    double fl = quot_rd((double)s, dm, dinv);
     double suml = group_psum<false>(g, fl);
     suml -= to_uint(suml);
     out.low = er_set_d(suml);

@@ -248,7 +248,7 @@ struct WaveStage {
 // `res`, RARE_RES_WIDTH ints per slot for the first res_cap slots of each sub-queue, so that the
 // rare pass reads 4n contiguous bytes per item instead of one cache line per residue row.  A
 // one-wave kernel after the rare pass clears the counters for the next call on the stream.
-// Evaluation, comparison, division and scaling share the queue of a (context, stream) pair, one
+// Evaluation, comparison and the division of long arrays share the queue of a (context, stream) pair, one
 // call at a time.
 constexpr int RARE_RES_WIDTH = 128;  // ints per staged slot: two numbers of up to 64 residues
 constexpr int RARE_SUBQ = 64;        // sub-queues
@@ -439,12 +439,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(N <= 32 ?
     }
 }
 
-// Any n <= 64: one group per number throughout.
-template <bool FAST>
-__global__ __launch_bounds__(BLOCK) void k_eval_group(const DevCtx *__restrict__ c, int G, const int *__restrict__ x,
+// One group of G lanes per number throughout: sets without a lane kernel (L = 0: up to G moduli), and short
+// calls of the others (L moduli), where this is one launch instead of three.
+template <int G, int L, bool FAST>
+__global__ __launch_bounds__(BLOCK) void k_eval_group(const DevCtx *__restrict__ c, const int *__restrict__ x,
                                                       long long smod, long long snum, long long count,
                                                       interval_t *__restrict__ out, int *__restrict__ status) {
-    Group g = make_group(G, c->n);
+    Group g = make_group(G, L ? L : c->n);
     const int P = 64 / G;
     long long wave = ((long long)blockIdx.x * BLOCK + threadIdx.x) >> 6;
     long long nwaves = ((long long)gridDim.x * BLOCK) >> 6;
@@ -769,12 +770,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(N <= 32 ?
     }
 }
 
-// Any n <= 64: one group per pair throughout.
-static __global__ __launch_bounds__(BLOCK) void k_cmp_group(const DevCtx *__restrict__ c, int G, const int *__restrict__ x,
-                                                     long long xsm, long long xsn, const int *__restrict__ y,
+// One group per pair throughout, as k_eval_group.
+template <int G, int L>
+__global__ __launch_bounds__(BLOCK) void k_cmp_group(const DevCtx *__restrict__ c, const int *__restrict__ x, long long xsm,
+                                                      long long xsn, const int *__restrict__ y,
                                                      long long ysm, long long ysn, long long count,
                                                      int *__restrict__ sign, int *__restrict__ status) {
-    Group g = make_group(G, c->n);
+    Group g = make_group(G, L ? L : c->n);
     const int P = 64 / G;
     long long wave = ((long long)blockIdx.x * BLOCK + threadIdx.x) >> 6;
     long long nwaves = ((long long)gridDim.x * BLOCK) >> 6;
@@ -806,7 +808,7 @@ struct DivLeaf {
     const int *s;
     template <int I>
     GRNS_HD double get() {
-        return UP ? ddiv_ru((double)s[I], c->dm[I]) : ddiv_rd((double)s[I], c->dm[I]);
+        return UP ? quot_ru((double)s[I], c->dm[I], c->dinv[I]) : quot_rd((double)s[I], c->dm[I], c->dinv[I]);
     }
 };
 // ... and for the main sums: dmul_rd / dmul_ru(s_i, RECIP_RD/RU) (src/rnseval.cuh:46-47).
@@ -1691,38 +1693,36 @@ GRNS_D bool div_words_ok(const DevCtx *c, const Group &g, int xi, int di) {
 // the word division never writes it).
 constexpr int DIV_MARK = (int)0x80000000u;
 
-// Division of the pairs div_words_ok accepts (group of GD lanes per pair); the others go to the
-// rare queue, and k_div_rare runs the reference loop for them.
+// Division, a group of GD lanes per pair: on words where div_words_ok accepts the pair, else by the reference
+// loop.
+template <int GD>
+GRNS_D void group_div_any(const DevCtx *c, const Group &g, int xi, int di, bool fast, int &q, int &r, int &st) {
+    if (div_words_ok(c, g, xi, di)) group_div_words<GD>(c, g, xi, di, q, r);
+    else if (fast) group_div<true>(c, g, xi, di, q, r, st);
+    else group_div<false>(c, g, xi, di, q, r, st);
+}
 template <int GD>
 __global__ __launch_bounds__(BLOCK) void k_div_words(const DevCtx *__restrict__ c, const int *__restrict__ x,
                                                      const int *__restrict__ d, long long smod, long long snum,
                                                      long long count, int *__restrict__ q, int *__restrict__ r,
-                                                     RareQ rq) {
+                                                     bool fast, int *__restrict__ status) {
     const Group g = make_group(GD, c->n);
     constexpr int P = 64 / GD;
     const long long wave = ((long long)xcd_block() * BLOCK + threadIdx.x) >> 6;
     const long long nwaves = ((long long)gridDim.x * BLOCK) >> 6;
     for (long long j0 = wave * P; j0 < count; j0 += nwaves * P) {
         const long long j = j0 + (threadIdx.x & 63) / GD;
-        const bool valid = j < count;
-        bool ok = false;
-        if (valid) {
+        if (j < count) {
             const bool act = g.gl < g.L;
             const long long off = j * snum + (long long)g.gl * smod;
-            const int xi = act ? x[off] : 0;
-            const int di = act ? d[off] : 0;
-            ok = div_words_ok(c, g, xi, di);
-            if (ok) {
-                int qq, rr;
-                group_div_words<GD>(c, g, xi, di, qq, rr);
-                if (act) {
-                    q[off] = qq;
-                    r[off] = rr;
-                }
+            int qq, rr, st = 0;
+            group_div_any<GD>(c, g, act ? x[off] : 0, act ? d[off] : 0, fast, qq, rr, st);
+            if (act) {
+                q[off] = qq;
+                r[off] = rr;
             }
+            if (g.gl == 0 && st) atomicOr(status, st);
         }
-        const bool rare = valid && !ok && g.gl == 0;
-        if (!rare_push(rq, rare, j)) q[j * snum] = DIV_MARK;
     }
 }
 
@@ -1987,8 +1987,7 @@ GRNS_D int group_scaling_step(const DevCtx *c, const Group &g, bool first, int j
     const double dinv = act ? c->dinv[g.gl] : 1.0;
     const int ci = act ? mulmod_recip(y, c->w[g.gl], mi, dinv) : 0;
     const int k = first ? group_rank(c, g, y, ci) : group_rank_fast(c, g, ci);
-    unsigned sum = act ? (unsigned)c->part_pow2_res[j - 1][g.gl] * (unsigned)ci : 0u;
-    for (int s = 1; s < g.G; s <<= 1) sum += (unsigned)__shfl_xor((int)sum, s, 64);
+    const unsigned sum = group_sum(g, act ? (unsigned)c->part_pow2_res[j - 1][g.gl] * (unsigned)ci : 0u);
     residue = (int)((sum - (unsigned)k * (unsigned)c->prod_pow2_res[j - 1]) & ((1u << j) - 1u));
     const int mult = psubmod(y, (int)rem_trunc_d((long long)residue, (double)residue, mi, dinv), mi, dinv);
     const int inv = act ? c->pow2_inv[j - 1][g.gl] : 0;

@@ -538,6 +538,32 @@ grns_status grns_ctx_status(grns_ctx *c, int *bits) {
     return GRNS_OK;
 }
 
+// Evaluations and comparisons of at most 64 waves of groups per CU take a wave group per number from the
+// start: one launch, where a lane per number needs a rare pass and its queue's reset behind it.  By
+// groups and by lanes, uniform numbers: 4096 of 64 moduli 8 and 13 us, at the line 8-15 and 13-16 us,
+// at twice the line 13-26 and 13-17 us; values near 0, which all need the refinement loop, 2048 of 32
+// moduli 15 and 24 us, at the line 76 and 97 us.
+static bool group_call(const grns_ctx *c, size_t count) {
+    return count * (size_t)groups_for(c->n) <= (size_t)4096 * (size_t)(c->cus > 0 ? c->cus : 256);
+}
+
+// The group kernel of G lanes for n moduli: LAUNCH(G, L), L = n where the set fills the group.
+#define GRNS_BY_GROUP(G, n, LAUNCH)                                                                              \
+    switch ((G) == (n) ? -(G) : (G)) {                                                                           \
+        case -1: case 1: LAUNCH(1, 1) break;                                                                     \
+        case -2: LAUNCH(2, 2) break;                                                                             \
+        case -4: LAUNCH(4, 4) break;                                                                             \
+        case 4: LAUNCH(4, 0) break;                                                                              \
+        case -8: LAUNCH(8, 8) break;                                                                             \
+        case 8: LAUNCH(8, 0) break;                                                                              \
+        case -16: LAUNCH(16, 16) break;                                                                          \
+        case 16: LAUNCH(16, 0) break;                                                                            \
+        case -32: LAUNCH(32, 32) break;                                                                          \
+        case 32: LAUNCH(32, 0) break;                                                                            \
+        case -64: LAUNCH(64, 64) break;                                                                          \
+        default: LAUNCH(64, 0) break;                                                                            \
+    }
+
 grns_status grns_eval(grns_ctx *c, const int *x, long long smod, long long snum, size_t count, grns_interval *out,
                       int fast, void *stream) {
     if (c && c->device < 0) return GRNS_ERR_ARG;
@@ -581,7 +607,7 @@ grns_status grns_eval(grns_ctx *c, const int *x, long long smod, long long snum,
         hipLaunchKernelGGL(k_rare_reset, dim3(1), dim3(64), 0, S(stream), q.ctr);                                \
         return launch_check();                                                                                   \
     }
-    switch (c->n) {
+    switch (group_call(c, count) ? 0 : c->n) {
         GRNS_EVAL_CASE(4)
         GRNS_EVAL_CASE(8)
         GRNS_EVAL_CASE(16)
@@ -601,8 +627,15 @@ grns_status grns_eval(grns_ctx *c, const int *x, long long smod, long long snum,
     }
     int G = groups_for(c->n);
     dim3 g2((unsigned)grid_groups(count, G));
-    if (fast) hipLaunchKernelGGL((k_eval_group<true>), g2, blk, 0, S(stream), c->d, G, x, smod, snum, cnt, o, c->d_status);
-    else hipLaunchKernelGGL((k_eval_group<false>), g2, blk, 0, S(stream), c->d, G, x, smod, snum, cnt, o, c->d_status);
+    const int tk = stage_begin(c, 0, stream);
+#define GRNS_EVAL_GROUP(GG, LL)                                                                                  \
+    if (fast) hipLaunchKernelGGL((k_eval_group<GG, LL, true>), g2, blk, 0, S(stream), c->d, x, smod, snum, cnt, o, \
+                                 c->d_status);                                                                   \
+    else hipLaunchKernelGGL((k_eval_group<GG, LL, false>), g2, blk, 0, S(stream), c->d, x, smod, snum, cnt, o,     \
+                            c->d_status);
+    GRNS_BY_GROUP(G, c->n, GRNS_EVAL_GROUP)
+#undef GRNS_EVAL_GROUP
+    stage_end(c, 0, tk, stream);
     return launch_check();
 }
 
@@ -636,7 +669,7 @@ grns_status grns_cmp(grns_ctx *c, const int *x, long long xsm, long long xsn, co
         hipLaunchKernelGGL(k_rare_reset, dim3(1), dim3(64), 0, S(stream), q.ctr);                                  \
         return launch_check();                                                                                     \
     }
-    switch (c->n) {
+    switch (group_call(c, count) ? 0 : c->n) {
         GRNS_CMP_CASE(4)
         GRNS_CMP_CASE(8)
         GRNS_CMP_CASE(16)
@@ -653,7 +686,13 @@ grns_status grns_cmp(grns_ctx *c, const int *x, long long xsm, long long xsn, co
     }
     int G = groups_for(c->n);
     dim3 g2((unsigned)grid_groups(count, G));
-    hipLaunchKernelGGL(k_cmp_group, g2, blk, 0, S(stream), c->d, G, x, xsm, xsn, y, ysm, ysn, cnt, sign, c->d_status);
+    const int tk = stage_begin(c, 1, stream);
+#define GRNS_CMP_GROUP(GG, LL)                                                                                     \
+    hipLaunchKernelGGL((k_cmp_group<GG, LL>), g2, blk, 0, S(stream), c->d, x, xsm, xsn, y, ysm, ysn, cnt, sign,      \
+                       c->d_status);
+    GRNS_BY_GROUP(G, c->n, GRNS_CMP_GROUP)
+#undef GRNS_CMP_GROUP
+    stage_end(c, 1, tk, stream);
     return launch_check();
 }
 
@@ -679,27 +718,35 @@ grns_status grns_div(grns_ctx *c, const int *x, const int *d, long long smod, lo
     long long cnt = (long long)count;
     // canonical pairs with d != 0: word division; the reference loop for the others (rare pass)
     const int GW = reference ? 0 : words_group(c);
-    if (GW) {
+    if (GW && count >= div_lanes_min(c)) {
         RareQ rq;
         grns_status qs = rare_queue(c, stream, rq);
         if (qs != GRNS_OK) return qs;
-        dim3 gw((unsigned)grid_groups(count, GW)), rg((unsigned)rare_grid(count));
-        if (count >= div_lanes_min(c)) {
-            qs = matrix_div(c, x, d, smod, snum, count, q, r, rq, S(stream));
-            if (qs != GRNS_OK) return qs;
-        } else switch (GW) {
-            case 2: hipLaunchKernelGGL((k_div_words<2>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-            case 4: hipLaunchKernelGGL((k_div_words<4>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-            case 8: hipLaunchKernelGGL((k_div_words<8>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-            case 16: hipLaunchKernelGGL((k_div_words<16>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-            case 32: hipLaunchKernelGGL((k_div_words<32>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-            default: hipLaunchKernelGGL((k_div_words<64>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, rq); break;
-        }
-        if (hipGetLastError() != hipSuccess) return GRNS_ERR_HIP;
+        dim3 rg((unsigned)rare_grid(count));
+        qs = matrix_div(c, x, d, smod, snum, count, q, r, rq, S(stream));
+        if (qs != GRNS_OK) return qs;
         if (fast) hipLaunchKernelGGL((k_div_rare<true>), rg, blk, 0, S(stream), c->d, G, x, d, smod, snum, cnt, q, r, c->d_status, rq);
         else hipLaunchKernelGGL((k_div_rare<false>), rg, blk, 0, S(stream), c->d, G, x, d, smod, snum, cnt, q, r, c->d_status, rq);
         if (hipGetLastError() != hipSuccess) return GRNS_ERR_HIP;
         hipLaunchKernelGGL(k_rare_reset, dim3(1), dim3(64), 0, S(stream), rq.ctr);
+        return launch_check();
+    }
+    if (GW) {
+        dim3 gw((unsigned)grid_groups(count, GW));
+#define GRNS_DIV_CASE(GG)                                                                                            \
+    case GG:                                                                                                         \
+        hipLaunchKernelGGL((k_div_words<GG>), gw, blk, 0, S(stream), c->d, x, d, smod, snum, cnt, q, r, fast,          \
+                           c->d_status);                                                                             \
+        break;
+        switch (GW) {
+            GRNS_DIV_CASE(2)
+            GRNS_DIV_CASE(4)
+            GRNS_DIV_CASE(8)
+            GRNS_DIV_CASE(16)
+            GRNS_DIV_CASE(32)
+            GRNS_DIV_CASE(64)
+        }
+#undef GRNS_DIV_CASE
         return launch_check();
     }
     if (fast) hipLaunchKernelGGL((k_div<true>), grid, blk, 0, S(stream), c->d, G, x, d, smod, snum, cnt, q, r, c->d_status);
