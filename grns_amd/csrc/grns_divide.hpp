@@ -211,22 +211,29 @@ GRNS_D void residue_rows(const MatTab &tab, const ModRec *rec, int lane, int n, 
 
 constexpr int div_waves(int NP) { return NP == 64 ? 2 : NP == 8 ? 4 : 3; }  // per SIMD: registers and LDS allow these
 
+// A block's LDS: digits of each wave's pairs, and the small tables.
 template <int NP>
-__global__ __launch_bounds__(BLOCK, div_waves(NP)) void k_div_mat(const DevCtx *__restrict__ c, MatTab tab,
-                                                                  const int *x, const int *d, long long smod,
-                                                                  long long snum, long long count, int *q, int *r,
-                                                                  RareQ rq) {
+struct DivShared {
+    int digits[BLOCK / 64][DivShape<NP>::ROWS * 64];
+    __align__(16) int init[Mat<NP>::DT * 32];
+    __align__(16) int mdig[8 * Mat<NP>::DT];
+    ModRec rec[NP];
+};
+
+// The wave's pairs j0 .. j0 + 63 (those below count; all waves of a block call it).  rest(left, j): the
+// lane's pair j if it is left to the reference loop (a residue outside [0, m), or a zero divisor).
+template <int NP, class Rest>
+GRNS_D void div_wave(const DevCtx *__restrict__ c, const MatTab &tab, DivShared<NP> &sh, const int *x, const int *d,
+                     long long smod, long long snum, long long count, long long j0, int *q, int *r, Rest rest) {
     constexpr int KR = Mat<NP>::KR, ND = Mat<NP>::ND, DT = Mat<NP>::DT;
-    __shared__ int digits[BLOCK / 64][DivShape<NP>::ROWS * 64];
-    __shared__ __align__(16) int init[DT * 32], mdig[8 * DT];
-    __shared__ ModRec rec[NP];
+    int *init = sh.init, *mdig = sh.mdig;
+    ModRec *rec = sh.rec;
     for (int i = threadIdx.x; i < DT * 32; i += BLOCK) init[i] = tab.crt7_init[i];
     for (int i = threadIdx.x; i < 8 * DT; i += BLOCK) mdig[i] = tab.m28[i];
     for (int i = threadIdx.x; i < NP; i += BLOCK) rec[i] = tab.rec[i];
     const int lane = threadIdx.x & 63, h = lane >> 5;
     const int n = c->n;
-    const long long j0 = ((long long)xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6)) * 64;
-    int *lds = digits[threadIdx.x >> 6], *own = lds + lane;
+    int *lds = sh.digits[threadIdx.x >> 6], *own = lds + lane;
     const bool quad = quads(x, smod, snum) && quads(d, smod, snum);
     DigitColumn col[2];
     const int *p[2];
@@ -374,7 +381,19 @@ __global__ __launch_bounds__(BLOCK, div_waves(NP)) void k_div_mat(const DevCtx *
         else if (full) residue_rows<NP, STORE_QUADS>(tab, rec, lane, n, B, any, on, dst, smod);
         else residue_rows<NP, STORE_ANY>(tab, rec, lane, n, B, any, on, dst, smod);
     }
-    if (!rare_push(rq, jl < count && !ok, jl)) q[jl * snum] = DIV_MARK;
+    rest(jl < count && !ok, jl);
+}
+
+template <int NP>
+__global__ __launch_bounds__(BLOCK, div_waves(NP)) void k_div_mat(const DevCtx *__restrict__ c, MatTab tab,
+                                                                  const int *x, const int *d, long long smod,
+                                                                  long long snum, long long count, int *q, int *r,
+                                                                  RareQ rq) {
+    __shared__ DivShared<NP> sh;
+    const long long j0 = ((long long)xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6)) * 64;
+    div_wave<NP>(c, tab, sh, x, d, smod, snum, count, j0, q, r, [&](bool left, long long j) {
+        if (!rare_push(rq, left, j)) q[j * snum] = DIV_MARK;
+    });
 }
 
 }  // namespace grns

@@ -6,7 +6,7 @@
 // and the steps read these four at a time, the same address in every lane.  The residues are loaded a
 // second time, now with the modulus as the lane, a register per number (16 bytes for four numbers
 // where the array allows); the results take the place of the words in LDS and leave together, a row of
-// numbers per modulus.  2^20 numbers of 64 moduli, exponents to 1900: 2.31 -> 0.88 ms, of which 0.31 ms
+// numbers per modulus.  2^20 numbers of 64 moduli, exponents to 1900: 2.31 -> 0.94 ms, of which 0.31 ms
 // are left at exponent 0; a step of 2^-30 of all of them takes 17 us, the rate at which its 47 vector
 // instructions per four steps (16 of them 32-bit multiplications) issue.  Numbers of 32, 16, 8
 // moduli: 0.93, 0.61, 0.26 -> 0.42, 0.17, 0.077 ms.
@@ -16,15 +16,23 @@
 
 namespace grns {
 
+// A block's LDS.
 template <int NP>
-__global__ __launch_bounds__(BLOCK, 4) void k_scale_mat(const DevCtx *__restrict__ c, MatTab tab, const int *x,
-                                                        long long smod, long long snum,
-                                                        const unsigned *__restrict__ D, long long count, int *y) {
+struct ScaleShared {
+    __align__(16) int init[Mat<NP>::WT * 32];
+    __align__(16) int mdig[8 * Mat<NP>::WT];
+    ModRec rec[NP];
+    unsigned words[BLOCK / 64][32 * (NP + 1)];
+    __align__(16) unsigned digits[BLOCK / 64][(64 / NP) * (2 * NP + 4)];  // four are read past the last
+};
+
+// The wave's numbers j0 .. j0 + 31 (those below count; all waves of a block call it).
+template <int NP>
+GRNS_D void scale_wave(const DevCtx *__restrict__ c, const MatTab &tab, ScaleShared<NP> &sh, const int *x, long long smod,
+                       long long snum, const unsigned *__restrict__ D, long long count, long long j0, int *y) {
     constexpr int WT = Mat<NP>::WT, KR = Mat<NP>::KR, S = NP + 1, GD = NP, K = NP / 2;  // K numbers per group
-    __shared__ __align__(16) int init[WT * 32], mdig[8 * WT];
-    __shared__ ModRec rec[NP];
-    __shared__ unsigned words[BLOCK / 64][32 * S];
-    __shared__ __align__(16) unsigned digits[BLOCK / 64][(64 / NP) * (2 * NP + 4)];  // four are read past the last
+    int *init = sh.init, *mdig = sh.mdig;
+    ModRec *rec = sh.rec;
     for (int i = threadIdx.x; i < WT * 32; i += BLOCK) init[i] = tab.crt8_init[i];
     for (int i = threadIdx.x; i < 8 * WT; i += BLOCK) mdig[i] = tab.m8[i];
     for (int i = threadIdx.x; i < NP; i += BLOCK) rec[i] = tab.rec[i];
@@ -34,8 +42,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_scale_mat(const DevCtx *__restrict
     const Group g = make_group(GD, n);
     const bool quad = quads(x, smod, snum);
     const bool rows = snum == 1 && (smod & 3) == 0 && ((uintptr_t)x & 15) == 0;
-    unsigned *st = words[threadIdx.x >> 6], *dp = digits[threadIdx.x >> 6] + (g.base / NP) * (2 * NP + 4);
-    const long long j0 = ((long long)xcd_block() * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 32;
+    unsigned *st = sh.words[threadIdx.x >> 6], *dp = sh.digits[threadIdx.x >> 6] + (g.base / NP) * (2 * NP + 4);
     if (j0 >= count) return;
     const long long jl = j0 + (lane & 31), jc = jl < count ? jl : count - 1;
     const int Dl = (int)D[jc];
@@ -107,6 +114,15 @@ __global__ __launch_bounds__(BLOCK, 4) void k_scale_mat(const DevCtx *__restrict
     } else if (jl < count) {
         for (int i = h; i < n; i += 2) y[jl * snum + (long long)i * smod] = (int)st[(lane & 31) * S + i];
     }
+}
+
+template <int NP>
+__global__ __launch_bounds__(BLOCK, 4) void k_scale_mat(const DevCtx *__restrict__ c, MatTab tab, const int *x,
+                                                        long long smod, long long snum,
+                                                        const unsigned *__restrict__ D, long long count, int *y) {
+    __shared__ ScaleShared<NP> sh;
+    const long long j0 = ((long long)xcd_block() * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 32;
+    scale_wave<NP>(c, tab, sh, x, smod, snum, D, count, j0, y);
 }
 
 }  // namespace grns
