@@ -585,6 +585,17 @@ GRNS_HD double psum_one(Leaf &leaf) {
     }
 }
 
+// The compiler's scheduler stops here: unrolled passes over tables and operands otherwise have the
+// loads of all of them in flight, and spill.
+GRNS_D void sched_stop() { __builtin_amdgcn_sched_barrier(0); }
+
+// Hides a per-lane pointer's value: offsets from it are not computed ahead of the caller's loop.
+GRNS_D const int *lane_point(const int *p) {
+    long long v = reinterpret_cast<long long>(p);
+    asm volatile("" : "+v"(v));
+    return reinterpret_cast<const int *>(v);
+}
+
 // Orders the wave's own LDS accesses: what any lane wrote before is read by every lane after.
 GRNS_D void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

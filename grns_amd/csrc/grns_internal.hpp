@@ -23,6 +23,7 @@ struct grns_ctx {
     unsigned *d_crt = nullptr;      // DevCtx::crt_words
     int max_blocks = 2048;         // arg-max stage-1 grid, from the occupancy query (max_grid_for)
     int max_blocks_occ = 2048;     // the same as set at context creation (test hooks restore it)
+    int max_blocks_nm = 1024;      // the most blocks of it over a number-major array (resident ones)
     // rare-item queues of the per-call eval / cmp kernels, one per stream (made on first use)
     struct RareQueue {
         void *stream;

@@ -1134,12 +1134,14 @@ GRNS_D void coop_resolve(const DevCtx *c, const int *__restrict__ x, long long s
 // stays unknown and the order is exact.  Refined keys lie near 0 or 1, so two keys that do not
 // overlap may belong to x near 0 and y near M; the difference certificates of lane_cmp_exact are
 // therefore only used for overlapping keys.
+// Not inlined, four loads in flight: one residue at a time, in registers beside the streaming loop,
+// each merge of such candidates took a load's latency per residue.
 template <int N>
-GRNS_D void refine_key(const DevCtx *c, const int *__restrict__ x, long long smod, long long snum, MaxCand &e) {
-    if (e.idx < 0 || e.lo >= 0) return;
+__device__ __attribute__((noinline)) MaxCand refined_key(const DevCtx *c, const int *__restrict__ x, long long smod,
+                                                         long long snum, MaxCand e) {
     const int *p = x + e.idx * snum;
     double A = 0.0, B = 0.0;
-#pragma unroll 1
+#pragma unroll 4
     for (int i = 0; i < N; i++) {
         const double dx = (double)p[(long long)i * smod];
         A += fract_d(dx * c->shi[i]);
@@ -1155,9 +1157,67 @@ GRNS_D void refine_key(const DevCtx *c, const int *__restrict__ x, long long smo
         e.lo = 1.0 - ((1.0 - H) + E) * s - 0x1p-52;
         e.hi = fmin(1.0, 1.0 - ((1.0 - H) - E) * s + 0x1p-52);
     }
+    return e;
+}
+template <int N>
+GRNS_D void refine_key(const DevCtx *c, const int *__restrict__ x, long long smod, long long snum, MaxCand &e) {
+    if (e.idx >= 0 && e.lo < 0) e = refined_key<N>(c, x, smod, snum, e);
 }
 
-constexpr int LANE_UNROLL = 1;  // the stage-1 loop keeps its occupancy: overlaps there are rare
+// Whether numbers a and b of x have the same residues, and, of two that do not, the order by their small
+// difference where it has one (as lane_cmp_exact), out of the streaming loop for the same reason, the
+// residues eight at a time.  A kernel has the registers of what it calls: the pointers are walked.
+template <int N>
+__device__ __attribute__((noinline)) bool lane_equal(const int *__restrict__ x, long long smod, long long snum,
+                                                     long long a, long long b) {
+    const int *pa = x + a * snum, *pb = x + b * snum;
+    int diff = 0;
+#pragma unroll 1
+    for (int i = 0; i < N && !diff; i += 4) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            diff |= *pa ^ *pb;
+            pa = lane_point(pa + smod);
+            pb = lane_point(pb + smod);
+        }
+    }
+    return diff == 0;
+}
+template <int N>
+__device__ __attribute__((noinline)) int lane_order(const DevCtx *c, const int *__restrict__ x, long long smod,
+                                                    long long snum, long long a, long long b) {
+    constexpr int U = N < 8 ? N : 8;
+    const int *pa = x + a * snum, *pb = x + b * snum;
+    const int m0 = c->m[0];
+    int t = (int)((unsigned)*pa - (unsigned)*pb);
+    if (t > m0 / 2) t -= m0;
+    else if (t <= -((m0 + 1) / 2)) t += m0;
+    const unsigned at = 2u * (unsigned)(t < 0 ? -t : t);
+    bool canon = true, small = true;
+#pragma unroll 1
+    for (int i0 = 0; i0 < N; i0 += U) {
+        int av[U], bv[U];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            av[k] = *pa;
+            bv[k] = *pb;
+            pa = lane_point(pa + smod);
+            pb = lane_point(pb + smod);
+        }
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int m = c->m[i0 + k];
+            canon &= (unsigned)av[k] < (unsigned)m && (unsigned)bv[k] < (unsigned)m;
+            int d = (int)((unsigned)av[k] - (unsigned)bv[k]);
+            d += (d < 0) ? m : 0;
+            const int tm = t + ((t < 0) ? m : 0);
+            small &= d == tm && (i0 + k == 0 || at < (unsigned)m);
+        }
+    }
+    if (!canon) return 2;
+    if (small) return (t > 0) - (t < 0);
+    return near_sign<1>(c, x + a * snum, smod, x + b * snum, smod);
+}
 
 // Every lane proposes (e -> best): keys decide, then the exact order (lowest index among equal
 // values).  All 64 lanes of the wave must call this.
@@ -1172,9 +1232,8 @@ GRNS_D void max_merge(const DevCtx *c, const int *__restrict__ x, long long smod
         d = max_decide(e, best);
     }
     int r = 0;
-    if (d == 2)
-        r = lane_cmp_exact<LANE_UNROLL>(c, x + e.idx * snum, smod, x + best.idx * snum, smod,
-                                        e.lo >= 0 && best.lo >= 0);
+    if (d == 2 && !lane_equal<N>(x, smod, snum, e.idx, best.idx))
+        r = e.lo >= 0 && best.lo >= 0 ? lane_order<N>(c, x, smod, snum, e.idx, best.idx) : 2;
     coop_resolve<N>(c, x, smod, snum, e.idx, best.idx, r);
     bool take = (d == 1) || (d == 2 && (r > 0 || (r == 0 && e.idx < best.idx)));
     if (take) best = e;
@@ -1262,6 +1321,28 @@ GRNS_D bool pivot_before(const MaxCand &a, const MaxCand &b) {
     return a.lo > b.lo || (a.lo == b.lo && a.idx < b.idx);
 }
 
+// Whether the residues of the wave's candidate base + lane are `pivot`'s: rows of the residue copies are
+// read side by side, 16 bytes per lane.  Equal maxima are common (2930 equal candidates of 32 moduli):
+// a lane that reads its own candidate's row touches a line per load, and stage 2 took 33 us on its one
+// CU; this way 33 -> 20 us.
+template <int N>
+GRNS_D bool rows_equal(const int *__restrict__ rows, int base, int nrows, const int *__restrict__ pivot) {
+    typedef int row4 __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int LPR = N / 4, R = 64 / LPR, STEPS = LPR;  // lanes per row, rows per load
+    const int lane = threadIdx.x & 63;
+    const row4 pv = *reinterpret_cast<const row4 *>(pivot + 4 * (lane % LPR));
+    bool eq = false;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const int k = base + s * R + lane / LPR;
+        const row4 v = *reinterpret_cast<const row4 *>(rows + (long long)(k < nrows ? k : 0) * N + 4 * (lane % LPR));
+        const unsigned long long ne = __ballot(v[0] != pv[0] || v[1] != pv[1] || v[2] != pv[2] || v[3] != pv[3]);
+        const int i = lane - s * R;
+        if (i >= 0 && i < R) eq = (ne >> (i * LPR) & ((1ull << LPR) - 1)) == 0;
+    }
+    return eq;
+}
+
 constexpr int FBLOCK = 1024;             // threads of the stage-2 block
 constexpr int MAX_FINAL_PER_THREAD = 8;  // stage 2 takes at most FBLOCK * 8 candidates
 constexpr int MAX_PIVOT_ROUNDS = 3;      // then a tree over the live candidates (bounded depth)
@@ -1333,7 +1414,9 @@ __global__ __launch_bounds__(FBLOCK) void k_max_final(const DevCtx *__restrict__
             e.idx = -1; e.lo = -1.0; e.hi = -1.0;
             if (mine) e = part[k];
             int r = -1;
+            const bool same = rows_equal<N>(part_res, (T & ~63) + t * FBLOCK, nparts, pres);
             if (mine && e.idx != P.idx && e.lo > P.hi) r = 1;  // the keys order them
+            else if (mine && e.idx != P.idx && same) r = 0;
             else if (mine && e.idx != P.idx && e.hi >= P.lo)  // overlapping keys: exact order
                 r = lane_cmp_exact<16>(c, part_res + (long long)k * N, 1, pres, 1, e.lo >= 0 && P.lo >= 0);
             coop_resolve<N>(c, x, smod, snum, e.idx, P.idx, r);

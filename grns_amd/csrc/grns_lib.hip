@@ -334,19 +334,28 @@ long long rare_grid(size_t count) {
 
 // Grid of the arg-max stage-1 kernel on the context's device: its resident blocks (occupancy query),
 // scaled where a larger grid measured faster.
-int max_grid_for(const grns_ctx *c) {
+int max_grid_for(const grns_ctx *c, int &nm) {
     int cus = 0, per = 0;
+    nm = 1024;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1)
         return 2048;
     hipError_t e = hipErrorInvalidValue;
+    int pnm = 0;
+#define GRNS_OCC_CASE(NN)                                                                                             \
+    case NN:                                                                                                        \
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<NN, LD_MM>, BLOCK, 0);                   \
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&pnm, k_max_partial<NN, LD_NM>, BLOCK, 0); \
+        break;
     switch (c->n) {
-        case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<4, LD_MM>, BLOCK, 0); break;
-        case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<8, LD_MM>, BLOCK, 0); break;
-        case 16: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<16, LD_MM>, BLOCK, 0); break;
-        case 32: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<32, LD_MM>, BLOCK, 0); break;
-        case 64: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_max_partial<64, LD_MM>, BLOCK, 0); break;
+        GRNS_OCC_CASE(4)
+        GRNS_OCC_CASE(8)
+        GRNS_OCC_CASE(16)
+        GRNS_OCC_CASE(32)
+        GRNS_OCC_CASE(64)
         default: break;
     }
+#undef GRNS_OCC_CASE
+    if (e == hipSuccess && pnm > 0) nm = cus * pnm;
     if (e != hipSuccess || per < 1) return 2048;
     // At n = 16 and 32 (7 resident blocks per CU) a grid of 1.75 resident waves streams faster than
     // one: 2979 instead of 1772 blocks over 2^24 numbers took 167 instead of 185 us (n = 16) and 328
@@ -464,7 +473,7 @@ grns_status grns_ctx_create(const int *moduli, int n, int device, grns_ctx **out
         grns_ctx_destroy(c);
         return GRNS_ERR_HIP;
     }
-    c->max_blocks = c->max_blocks_occ = max_grid_for(c);
+    c->max_blocks = c->max_blocks_occ = max_grid_for(c, c->max_blocks_nm);
     if (scratch_setup(c->device) != GRNS_OK) {
         grns_ctx_destroy(c);
         return GRNS_ERR_HIP;
@@ -921,6 +930,12 @@ static grns_status max_run(grns_ctx *c, const int *x, long long smod, long long 
                            long long *out_idx, MaxCand *part, int *part_res, long long nb, long long ch, void *stream,
                            bool timed) {
     const bool mm = snum == 1 && count <= ((size_t)1 << 29);
+    // number-major arrays: fewer blocks are resident (LDS), and a grid of just over one or two times those
+    // leaves the last ones alone on the chip
+    if (!mm && smod == 1 && c->max_blocks == c->max_blocks_occ && nb > c->max_blocks_nm) {
+        ch = (((long long)count + c->max_blocks_nm - 1) / c->max_blocks_nm + BLOCK - 1) / BLOCK * BLOCK;
+        nb = ((long long)count + ch - 1) / ch;
+    }
     dim3 grid((unsigned)nb), blk(BLOCK), fblk(FBLOCK);
     long long cnt = (long long)count;
     int tk = -1;

@@ -82,17 +82,6 @@ GRNS_D v16i load_init(const int *p) {
 GRNS_D int other_half(int v) { return __shfl_xor(v, 32, 64); }
 GRNS_D double other_half_d(double v) { return __shfl_xor(v, 32, 64); }
 
-// The compiler's scheduler stops here: unrolled passes over tables and operands otherwise have the
-// loads of all of them in flight, and spill.
-GRNS_D void sched_stop() { __builtin_amdgcn_sched_barrier(0); }
-
-// Hides a per-lane pointer's value: offsets from it are not computed ahead of the caller's loop.
-GRNS_D const int *lane_point(const int *p) {
-    long long v = reinterpret_cast<long long>(p);
-    asm volatile("" : "+v"(v));
-    return reinterpret_cast<const int *>(v);
-}
-
 // Whether four residues of consecutive moduli of one number are one aligned 16-byte word (number-major
 // arrays whose number stride is a multiple of 4).
 GRNS_D bool quads(const int *x, long long smod, long long snum) {
