@@ -86,11 +86,12 @@ grns_status matrix_to_binary(grns_ctx *c, const int *x, long long smod, long lon
 grns_status matrix_from_binary(grns_ctx *c, const unsigned *w, long long wst, long long wsn, int nwords, const int *sign,
                                size_t count, int *x, long long smod, long long snum, hipStream_t s);
 // Divisions of at least this many pairs take a lane per pair (grns_divide.hip), shorter ones a wave
-// group per pair: 64 pairs to a wave leave the chip idle below.  Divisors of uniform length: 16384 pairs
-// of 8, 16, 32, 64 moduli take 19, 36, 54, 93 us by groups and 18, 23, 38, 82 us by lanes; the groups'
-// time falls with the quotient's length, to 16, 21, 26, 45 us for divisors as long as the dividend
-// (16, 19, 30, 57 us by lanes), hence the higher line above 16 moduli.
-inline size_t div_lanes_min(const grns_ctx *c) { return c->n > 16 ? 32768 : 16384; }
+// group per pair: 64 pairs to a wave leave the chip idle below.  By groups and by lanes: 16384 pairs with
+// divisors of uniform length 14 and 18 us (8 moduli), 34 and 24 us (16), 54 and 38 us (32), 103 and 82 us
+// (64), with divisors as long as the dividend 12 and 16, 18 and 18, 22 and 30, 46 and 57 us; 32768 pairs of
+// 32 moduli 91 and 40, 39 and 30 us, of 64 moduli 189 and 85, 84 and 57 us, of 8 moduli 25 and 18, 16 and
+// 17 us.  Hence a higher line for the sets whose short quotients the groups finish sooner.
+inline size_t div_lanes_min(const grns_ctx *c) { return c->n > 16 ? 32768 : c->n > 8 ? 16384 : 22528; }
 
 // Lane-per-pair division (grns_divide.hip): pairs it does not take go to the rare queue.
 grns_status matrix_div(grns_ctx *c, const int *x, const int *d, long long smod, long long snum, size_t count, int *q,
